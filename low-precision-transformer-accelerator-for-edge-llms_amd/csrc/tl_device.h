@@ -402,8 +402,8 @@ TL_DEV int sdot4x4(int4 a, int4 b, int acc) {
 }
 
 // v[0] + v[1] + ... + v[n-1] added in index order, starting from 0 (the
-// softmax denominator over block sums); up to 32 values are read before the
-// first add, so the chain costs one LDS latency instead of n
+// softmax denominator over block sums); 32 values are read before their first
+// add, so the chain costs one LDS latency per 32 values instead of n
 TL_DEV float ordered_sum(const float* v, int n) {
     float t = 0.0f;
     if (n <= 32) {
@@ -415,7 +415,14 @@ TL_DEV float ordered_sum(const float* v, int n) {
             if (i < n) t = t + r[i];
         return t;
     }
-    for (int i = 0; i < n; i++) t = t + v[i];
+    for (int i0 = 0; i0 < n; i0 += 32) {
+        float r[32];
+#pragma unroll
+        for (int i = 0; i < 32; i++) r[i] = v[min(i0 + i, n - 1)];
+#pragma unroll
+        for (int i = 0; i < 32; i++)
+            if (i0 + i < n) t = t + r[i];
+    }
     return t;
 }
 

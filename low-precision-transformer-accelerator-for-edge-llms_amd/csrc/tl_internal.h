@@ -262,7 +262,6 @@ hipError_t launch_argmax_tiles(hipStream_t s, const unsigned long long* part, in
                                unsigned long long* keys);
 hipError_t init_kernels();
 hipError_t init_decode_kernels();
-hipError_t init_prefill_kernels();
 hipError_t init_skinny_kernels();
 hipError_t launch_fill_u32(hipStream_t s, unsigned* p, int32_t n, unsigned v);
 hipError_t launch_causal_mask_i32(hipStream_t s, const int32_t* scores, int32_t rows, int32_t cols, int32_t qb,

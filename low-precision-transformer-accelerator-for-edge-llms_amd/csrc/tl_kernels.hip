@@ -932,22 +932,14 @@ __global__ __launch_bounds__(256) void attention_kernel(const int8_t* __restrict
 
 // ---------------------------------------------------------------------------
 // prefill attention on i8 MFMA (v_mfma_i32_32x32x32_i8), same arithmetic as
-// attention_kernel: one workgroup (4 wavefronts) per (query head, tile of 32
-// consecutive rows of one sequence at positions pos0 + r).  The INT8 cache
-// layouts are the MFMA operand fragments: lane l of a K fragment holds 16
-// dimensions of key l % 32 (one 16-byte chunk of the K plane), lane l of a V
-// fragment 16 keys of dimension l % 32 (one chunk of the V plane).  In the
-// 32 x 32 output lane l, register i holds row 8 (i / 4) + 4 (l / 32) + i % 4
-// and key (or dimension) l % 32.
-//   pass A  S = Q K^T per 32-key tile, row maxima over each row's keys
-//   pass B  exponentials; a 64-key block is two tiles, so the block-64
-//           butterfly is the sum of the two tiles' values (distance 32) and
-//           then lane distances 16 .. 1 -- the order of the decode kernels;
-//           row totals in block order
-//   pass C  p8 = rne(127 e / total) into LDS (rows x keys)
-//   pass D  O = P8 . V per 32-key chunk, integer partials added in LDS
-// Scores are recomputed per pass (K is an L2 hit), so LDS does not grow with
-// the context beyond the INT8 probabilities.
+// attention_kernel: one workgroup per (query head, tile of 32 consecutive rows
+// of one sequence at positions pos0 + r).  The INT8 cache layouts are the MFMA
+// operand fragments: lane l of a K fragment holds 16 dimensions of key l % 32
+// (one 16-byte chunk of the K plane), lane l of a V fragment 16 keys of
+// dimension l % 32 (one chunk of the V plane).  In a 32 x 32 output lane l,
+// register i holds row 8 (i / 4) + 4 (l / 32) + i % 4 of the A operand and row
+// l % 32 of the B operand.  attention_tile_reg_kernel (at most one 64-key block
+// per wavefront) keeps scores in registers, attention_tile_kernel recomputes them.
 // ---------------------------------------------------------------------------
 struct AttnTileArgs {
     const int8_t* q8;        // [rows][D]
@@ -1016,11 +1008,57 @@ TL_DEV double tile_q_scale(const AttnTileArgs& p, int r) {
     return p.qf ? quant_scale(__uint_as_float(p.qmax[(int64_t)r * kQmaxStride])) : p.q_scale[r];
 }
 
-__global__ __launch_bounds__(256) void attention_tile_kernel(AttnTileArgs p) {
+// ---------------------------------------------------------------------------
+// Prefill attention past the keys attention_tile_reg_kernel holds in
+// registers: one workgroup of NW wavefronts per (query head, tile of 32
+// consecutive rows), the same arithmetic, in the transposed layout
+// S^T = K Q^T (lane l: query row l % 32; register i: key 8 (i / 4) +
+// 4 (l / 32) + i % 4 of a 32-key tile), so that a row's scale, maximum, total
+// and last key are one value per lane.  Wavefront w owns the 64-key blocks
+// w, w + NW, ...; scores are recomputed by MFMA in each of three passes.
+//   pass A  each row's largest INT32 score: the score scale is positive, so
+//           f32(S) rs is monotone in S and the maximum of the products is the
+//           product of the maximum (half an instruction per key, v_max3)
+//   pass B  exponentials and block sums (as attention_tile_reg_kernel)
+//   pass C  probabilities and P . V.  rne(127 e / total) is 0 for every key
+//           below a score that follows from the row's maximum and total, and at
+//           most 254 keys of a row are not, so a 32-key tile or a group of four
+//           keys whose lanes all lie below it costs its maxima only.  Two
+//           v_permlane32_swap turn a lane's four packed words into the A
+//           fragment of P . V: probabilities never pass through LDS.
+// What bounds it: vector issue in pass B (about 18 instructions per key and
+// row for the exponential and its sum, 35 us of a 2048-token layer's 32
+// heads).  A 2048-token layer (32 heads) takes 74 us where the row layout with a second
+// exponential per key and probabilities in LDS took 206; 333 rows behind 701
+// keys 24 us against 51.
+// ---------------------------------------------------------------------------
+
+// a score S for which f32(S) rs - m < log(0.0039 total) - 1e-3 has probability
+// byte 0: e / total < 0.0039 (1 + 2^-20), where 127 e / total < 0.4954 rounds
+// to 0.  The threshold is formed in float32 with two whole steps of S to
+// spare over its rounding (|S| <= 64 127 127 < 2^20); a scale that is not a
+// positive normal number, or a NaN on the way, gives a threshold no score is below.
+TL_DEV int prob_zero_below(float m, float total, float rs) {
+    const float lim = m + (__logf(0.0039f * total) - 1e-3f);
+    const float s = fminf(fmaxf(lim / rs, -2097152.0f), 2097152.0f) - 2.0f;
+    return rs >= 0x1p-100f && rs <= 0x1p100f ? (int)s : -2147483647 - 1;
+}
+
+// the A fragment of P . V (row l % 32, keys 16 (l / 32) .. + 15 of a 32-key
+// tile) from the lane's words of four probabilities: word q holds keys
+// 8 q + 4 (l / 32) .. + 3, so words 0 and 2, 1 and 3 trade halves
+TL_DEV v4i prob_frag(const unsigned* w) {
+    const auto s02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+    const auto s13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+    return (v4i){(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
+}
+
+template <int NW>
+__global__ __launch_bounds__(NW * 64, 4) void attention_tile_kernel(AttnTileArgs p) {
     extern __shared__ __align__(16) int8_t tile_lds[];
     __shared__ __align__(16) int8_t qs8[32 * 64];   // Q quantized by the workgroup (float32 Q input)
-    __shared__ float scl[32], mrow[32], tot[32];
-    __shared__ float wmax[4][32];
+    __shared__ float scl[32];
+    __shared__ int wmax[NW][32];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const int col = lane & 31, hi = lane >> 5;
     const int h = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * 32;   // the longest (last) tiles dispatch first
@@ -1028,133 +1066,136 @@ __global__ __launch_bounds__(256) void attention_tile_kernel(AttnTileArgs p) {
     const int nr = min(32, p.rows - r0);
     const int pos_first = p.pos0 + r0;
     const int T = pos_first + nr;                  // the tile's last row sees keys 0 .. T - 1
-    const int tpad = (T + 63) & ~63, nblk = tpad >> 6;
-    int8_t* p8 = tile_lds;                         // [32][tpad]
-    float* bsum = (float*)(tile_lds + 32 * tpad);  // [32][nblk]
-    int* accs = (int*)(bsum + 32 * nblk);          // [32][64]
+    const int nblk = (T + 63) >> 6, bstride = nblk | 1;   // an odd row stride spreads the rows over the banks
+    int* accs = (int*)tile_lds;                    // [32][64]
+    float* bsum = (float*)(accs + 32 * 64);        // [32][bstride]
     const int D = p.n_heads * kHeadDim;
     const int64_t pl = p.kv.plane(p.seq, p.layer, g);
-    const int8_t* kp = p.kv.k + pl;
-    const int8_t* vp = p.kv.v + pl;
+    const int8_t* kp = p.kv.k + pl + hi * 1024 + col * 16;
+    const int8_t* vp = p.kv.v + pl + hi * 1024 + col * 16;
     const float sk = p.kv_sk[p.layer * p.n_kv + g], sv = p.kv_sv[p.layer * p.n_kv + g];
 
-    // Q fragments (rows past the tile's last read a stand-in, never stored)
     TileQ tq;
-    tile_q_load(p, r0, nr, h, col, hi, tq);
+    if (!p.qf || tid < 256) tile_q_load(p, r0, nr, h, col, hi, tq);
     if (tid < 32) scl[tid] = (float)((tile_q_scale(p, r0 + min(tid, nr - 1)) * (double)sk) * p.attn_scale);
-    for (int e = tid; e < 32 * 64; e += 256) accs[e] = 0;
-    tile_q_quantize(p, tq, qs8);
+    for (int e = tid; e < 32 * 64; e += NW * 64) accs[e] = 0;
+    if (tid < 256) tile_q_quantize(p, tq, qs8);
+    // K fragments of the wavefront's next block (two 32-key tiles), loaded one
+    // block ahead; past the last block the last is loaded again (in bounds)
+    v4i kf[4];
+    auto k_load = [&](int b) {
+        const int8_t* kb = kp + (int64_t)min(b, nblk - 1) * 4096;
+        kf[0] = ld16(kb);
+        kf[1] = ld16(kb + 2048);
+        kf[2] = ld16(kb + 512);
+        kf[3] = ld16(kb + 2560);
+    };
+    k_load(wave);
     __syncthreads();
     tile_q_frags(p, qs8, col, hi, tq);
     const v4i qa0 = tq.qa0, qa1 = tq.qa1;
-    float rs[16];
-    int rpos[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int r = 8 * (i >> 2) + 4 * hi + (i & 3);
-        rs[i] = scl[r];
-        rpos[i] = pos_first + r;
-    }
-    auto scores = [&](int kt) {
-        const int t = kt * 32 + col;
-        const int8_t* kb = kp + (int64_t)(t >> 6) * 4096 + hi * 1024 + (t & 63) * 16;
-        const v4i k0 = ld16(kb), k1 = ld16(kb + 2048);
-        v16i acc = {};
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(qa0, k0, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(qa1, k1, acc, 0, 0, 0);
-        return acc;
+    const float rs = scl[col];
+    const int rpos = pos_first + col;
+    v16i S0, S1;   // scores of the current block's two tiles
+    auto scores = [&](int next) {
+        const v4i k0 = kf[0], k1 = kf[1], k2 = kf[2], k3 = kf[3];
+        k_load(next);
+        S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k0, qa0, (v16i){}, 0, 0, 0);
+        S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k2, qa0, (v16i){}, 0, 0, 0);
+        S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k1, qa1, S0, 0, 0, 0);
+        S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k3, qa1, S1, 0, 0, 0);
     };
+    const int last = wave + (nblk - 1 - wave) / NW * NW;   // the wavefront's last block (if any)
 
-    // pass A: row maxima
-    float mx[16];
+    // pass A: each row's largest score
+    int mxs = -2147483647 - 1;
+    for (int b = wave; b < nblk; b += NW) {
+        scores(b == last ? wave : b + NW);
+        if (64 * b + 63 <= pos_first) {   // every row sees the whole block
 #pragma unroll
-    for (int i = 0; i < 16; i++) mx[i] = -INFINITY;
-    for (int b = wave; b < nblk; b += 4) {
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            const int kt = 2 * b + half, t = kt * 32 + col;
-            const v16i S = scores(kt);
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-                if (t <= rpos[i]) mx[i] = fmaxf(mx[i], (float)S[i] * rs[i]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        float v = mx[i];
-        v = half_max_f32(v);
-        if (col == 0) wmax[wave][8 * (i >> 2) + 4 * hi + (i & 3)] = v;
-    }
-    __syncthreads();
-    if (tid < 32) mrow[tid] = fmaxf(fmaxf(wmax[0][tid], wmax[1][tid]), fmaxf(wmax[2][tid], wmax[3][tid]));
-    __syncthreads();
-    float m[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) m[i] = mrow[8 * (i >> 2) + 4 * hi + (i & 3)];
-
-    // pass B: block sums
-    for (int b = wave; b < nblk; b += 4) {
-        const v16i S0 = scores(2 * b), S1 = scores(2 * b + 1);
-        const int t0 = 64 * b + col, t1 = t0 + 32;
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const float e0 = t0 <= rpos[i] ? tl_expf((float)S0[i] * rs[i] - m[i]) : 0.0f;
-            const float e1 = t1 <= rpos[i] ? tl_expf((float)S1[i] * rs[i] - m[i]) : 0.0f;
-            float v = e0 + e1;
-            v = half_butterfly_sum(v);
-            if (col == 0) bsum[(8 * (i >> 2) + 4 * hi + (i & 3)) * nblk + b] = v;
-        }
-    }
-    __syncthreads();
-    if (tid < 32) {
-        const float total = ordered_sum(bsum + tid * nblk, nblk);
-        tot[tid] = total;
-    }
-    __syncthreads();
-
-    // pass C: INT8 probabilities (zero past each row's last key): exponential
-    // / total correctly rounded, from each row's reciprocal and two residual
-    // corrections (e <= 1 <= total keeps e y finite; every total lies in
-    // [1, keys], the quotient's range, which the wave vote confirms)
-    float ty[16], tv[16];
-    bool in_range = true;
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        tv[i] = tot[8 * (i >> 2) + 4 * hi + (i & 3)];
-        ty[i] = __fdiv_rn(1.0f, tv[i]);
-        in_range = in_range && fabsf(tv[i]) >= 0x1p-64f && fabsf(tv[i]) <= 0x1p64f;
-    }
-    const bool fast = __all(in_range);
-    for (int b = wave; b < nblk; b += 4) {
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            const int kt = 2 * b + half, t = kt * 32 + col;
-            const v16i S = scores(kt);
+            for (int i = 0; i < 16; i++) mxs = max(mxs, max(S0[i], S1[i]));
+        } else {
+            const int t0 = 64 * b + 4 * hi;
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const int r = 8 * (i >> 2) + 4 * hi + (i & 3);
-                int8_t pq = 0;
-                if (t <= rpos[i]) {
-                    const float e = tl_expf((float)S[i] * rs[i] - m[i]);
-                    const float q = fast ? rn_div_fast(e, RnDiv{tv[i], ty[i], true}) : __fdiv_rn(e, tv[i]);
-                    float pr = __builtin_rintf(q * 127.0f);
-                    pr = pr < 0.0f ? 0.0f : (pr > 127.0f ? 127.0f : pr);
-                    pq = (int8_t)(int)pr;
-                }
-                p8[r * tpad + t] = pq;
+                const int t = t0 + 8 * (i >> 2) + (i & 3);
+                mxs = t <= rpos ? max(mxs, S0[i]) : mxs;
+                mxs = t + 32 <= rpos ? max(mxs, S1[i]) : mxs;
             }
         }
     }
+    mxs = max(mxs, lane_xor<32>(mxs));
+    if (hi == 0) wmax[wave][col] = mxs;
     __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; w++) mxs = max(mxs, wmax[w][col]);
+    const float m = (float)mxs * rs;
 
-    // pass D: O = P8 . V
+    // pass B: exponentials and block sums in the butterfly order
+    for (int b = wave; b < nblk; b += NW) {
+        scores(b == last ? wave : b + NW);
+        float a[16];   // token distance 32: the two tiles
+        if (64 * b + 63 <= pos_first) {
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                a[i] = tl_expf_nonpos((float)S0[i] * rs - m) + tl_expf_nonpos((float)S1[i] * rs - m);
+        } else {
+            const int t0 = 64 * b + 4 * hi;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int t = t0 + 8 * (i >> 2) + (i & 3);
+                const float e0 = t <= rpos ? tl_expf_nonpos((float)S0[i] * rs - m) : 0.0f;
+                const float e1 = t + 32 <= rpos ? tl_expf_nonpos((float)S1[i] * rs - m) : 0.0f;
+                a[i] = e0 + e1;
+            }
+        }
+        float d[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float b0 = a[r] + a[r + 8], b1 = a[r + 4] + a[r + 12];   // distance 16
+            d[r] = pair_sum<32>(b0 + b1);                                  // distances 8, 4
+        }
+        const float f = (d[0] + d[2]) + (d[1] + d[3]);                     // distances 2, 1
+        if (hi == 0) bsum[col * bstride + b] = f;
+    }
+    __syncthreads();
+    const float total = ordered_sum(bsum + col * bstride, nblk);
+
+    // pass C: INT8 probabilities (exponential / total correctly rounded, see
+    // attention_tile_reg_kernel; zero past the row's last key) and P . V
+    const RnDiv dv{total, __fdiv_rn(1.0f, total), true};
+    const bool fast = __all(fabsf(total) >= 0x1p-64f && fabsf(total) <= 0x1p64f);
+    const int thr = prob_zero_below(m, total, rs);
     v16i o0 = {}, o1 = {};
-    for (int kc = wave; kc < tpad / 32; kc += 4) {
-        const v4i a = *(const v4i*)(p8 + col * tpad + kc * 32 + hi * 16);
-        const int8_t* vb = vp + (int64_t)(kc * 2 + hi) * 1024 + col * 16;
-        const v4i b0 = ld16(vb), b1 = ld16(vb + 512);
-        o0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b0, o0, 0, 0, 0);
-        o1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b1, o1, 0, 0, 0);
+    auto pv = [&](const v16i& S, int kt) {   // keys 32 kt ..
+        int mt = max(S[0], S[1]);
+#pragma unroll
+        for (int i = 2; i < 16; i++) mt = max(mt, S[i]);
+        if (__builtin_amdgcn_ballot_w64(mt >= thr) == 0) return;
+        const int8_t* vb = vp + (int64_t)kt * 2048;
+        const v4i v0 = ld16(vb), v1 = ld16(vb + 512);
+        unsigned w[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            w[q] = 0;
+            const int mq = max(max(S[4 * q], S[4 * q + 1]), max(S[4 * q + 2], S[4 * q + 3]));
+            if (__builtin_amdgcn_ballot_w64(mq >= thr) == 0) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int t = 32 * kt + 8 * q + 4 * hi + r;
+                const float e = t <= rpos ? tl_expf_nonpos((float)S[4 * q + r] * rs - m) : 0.0f;
+                const float pr = __builtin_rintf((fast ? rn_div_fast(e, dv) : __fdiv_rn(e, total)) * 127.0f);
+                w[q] = __builtin_amdgcn_cvt_pk_u8_f32(pr, r, w[q]);
+            }
+        }
+        const v4i pa = prob_frag(w);
+        o0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(pa, v0, o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(pa, v1, o1, 0, 0, 0);
+    };
+    for (int b = wave; b < nblk; b += NW) {
+        scores(b + NW);
+        pv(S0, 2 * b);
+        pv(S1, 2 * b + 1);
     }
 #pragma unroll
     for (int i = 0; i < 16; i++) {
@@ -1164,7 +1205,7 @@ __global__ __launch_bounds__(256) void attention_tile_kernel(AttnTileArgs p) {
     }
     __syncthreads();
     const float pv_mult = deq_mult(1.0 / 127.0, sv);
-    for (int e = tid; e < 32 * 64; e += 256) {
+    for (int e = tid; e < 32 * 64; e += NW * 64) {
         const int r = e >> 6, d = e & 63;
         if (r < nr) p.out[(int64_t)(r0 + r) * D + (int64_t)h * kHeadDim + d] = (float)accs[e] * pv_mult;
     }
@@ -2070,213 +2111,148 @@ hipError_t launch_qkv_post(hipStream_t s, const float* qkv, int32_t rows, int32_
     return hipGetLastError();
 }
 
-// INT8 probabilities of 32 rows x tpad keys, block sums, partial sums
-static size_t tile_lds_bytes(int tpad) { return (size_t)32 * tpad + (size_t)32 * (tpad / 64) * sizeof(float) + 32 * 64 * sizeof(int); }
+// attention_tile_kernel: partial sums, block sums
+static size_t tile_lds_bytes(int nblk) { return (size_t)32 * 64 * sizeof(int) + (size_t)32 * (nblk | 1) * sizeof(float); }
 
-hipError_t init_prefill_kernels() {
-    return hipFuncSetAttribute((const void*)attention_tile_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)tile_lds_bytes(kTileMaxKeys));
-}
-
-// the same computation for contexts of at most 128 NB keys per wavefront
-// (NB blocks of 64 each, i.e. tpad <= 256 NB), in the transposed layout
-// S^T = K Q^T: lane l owns query row l % 32 and register i key
-// 8 (i / 4) + 4 (l / 32) + i % 4 of a 32-key tile.  A row's maximum is then
-// an in-lane maximum and one exchange with lane l ^ 32; of the block-64
-// butterfly (token distances 32, 16, 8, 4, 2, 1) only distance 4 (lane
-// l ^ 32) crosses lanes, the others add registers of one lane; four
-// probabilities of a lane are consecutive keys and leave as one 32-bit LDS
-// store.  Every K and V fragment of the wavefront is requested at the start;
-// scores and exponentials stay in registers across the passes.
-template <int NB>
-__global__ __launch_bounds__(256) void attention_tile_reg_kernel(AttnTileArgs p) {
-    extern __shared__ __align__(16) int8_t tile_lds[];
-    __shared__ __align__(16) int8_t qs8[32 * 64];   // Q quantized by the workgroup (float32 Q input)
-    __shared__ float scl[32], tot[32];
-    __shared__ float wmax[4][32];
+// The same computation for contexts of at most 64 NW keys: wavefront w of the
+// NW owns the one 64-key block w, so scores, exponentials and probabilities
+// stay in its registers across the passes, and its K and V fragments are all
+// requested at the start.  Layout as in attention_tile_kernel: a row's maximum
+// is an in-lane maximum and one exchange with lane l ^ 32; of the block-64
+// butterfly (token distances 32, 16, 8, 4, 2, 1) only distance 4 (lane l ^ 32)
+// crosses lanes, the others add registers of one lane.  512 rows from key 0:
+// 12.4 us per launch with one block per wavefront (8 wavefronts), where 4
+// wavefronts of two blocks and probabilities through LDS took 13.9.
+template <int NW>
+__global__ __launch_bounds__(NW * 64, 4) void attention_tile_reg_kernel(AttnTileArgs p) {
+    __shared__ int accs[32 * 64];
+    __shared__ __align__(16) float bsum[32 * (NW + 1)];   // an odd row stride spreads the rows over the banks
+    __shared__ __align__(16) int8_t qs8[32 * 64];         // Q quantized by the workgroup (float32 Q input)
+    __shared__ float scl[32];
+    __shared__ int wmax[NW][32];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const int col = lane & 31, hi = lane >> 5;
     const int h = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * 32;   // the longest (last) tiles dispatch first
     const int G = p.n_heads / p.n_kv, g = h / G;
     const int nr = min(32, p.rows - r0);
     const int pos_first = p.pos0 + r0;
-    const int T = pos_first + nr;
-    const int tpad = (T + 63) & ~63, nblk = tpad >> 6;
-    int8_t* p8 = tile_lds;                         // [32][tpad]
-    float* bsum = (float*)(tile_lds + 32 * tpad);  // [32][nblk]
-    int* accs = (int*)(bsum + 32 * nblk);          // [32][64]
+    const int T = pos_first + nr, nblk = (T + 63) >> 6;
     const int D = p.n_heads * kHeadDim;
-    const int64_t pl = p.kv.plane(p.seq, p.layer, g);
-    const int8_t* kp = p.kv.k + pl;
-    const int8_t* vp = p.kv.v + pl;
+    const int64_t pl = p.kv.plane(p.seq, p.layer, g) + (int64_t)min(wave, nblk - 1) * 4096 + hi * 1024 + col * 16;
     const float sk = p.kv_sk[p.layer * p.n_kv + g], sv = p.kv_sv[p.layer * p.n_kv + g];
+    const bool mine = wave < nblk;   // uniform; a wavefront without a block re-reads the last one, in bounds
 
-    // every load first: Q, then K of this wavefront's blocks b = wave + 4 j
-    // (two 32-key tiles each), then V of its 32-key chunks c = wave + 4 j.
-    // Blocks and chunks past the tile's keys (b >= nblk, c >= tpad / 32: a
-    // short causal tile) are skipped here and in every pass below -- each
-    // test is uniform per wavefront -- so a short tile costs less than the
-    // longest instead of the same.
     TileQ tq;
-    tile_q_load(p, r0, nr, h, col, hi, tq);
-    v4i kf[NB][2][2], vf[2 * NB][2];
+    if (!p.qf || tid < 256) tile_q_load(p, r0, nr, h, col, hi, tq);
+    v4i kf[4], vf[4];
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-        if (wave + 4 * j >= nblk) continue;
+    for (int i = 0; i < 4; i++) kf[i] = ld16(p.kv.k + pl + (i >> 1) * 512 + (i & 1) * 2048);   // [tile][dims 32 ..]
 #pragma unroll
-        for (int half = 0; half < 2; half++) {
-            const int t = 64 * (wave + 4 * j) + 32 * half + col;
-            const int8_t* kb = kp + (int64_t)(t >> 6) * 4096 + hi * 1024 + (t & 63) * 16;
-            kf[j][half][0] = ld16(kb);
-            kf[j][half][1] = ld16(kb + 2048);
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < 2 * NB; j++) {
-        const int kc = wave + 4 * j;
-        if (kc >= tpad / 32) continue;
-        const int8_t* vb = vp + (int64_t)(kc * 2 + hi) * 1024 + col * 16;
-        vf[j][0] = ld16(vb);
-        vf[j][1] = ld16(vb + 512);
-    }
+    for (int i = 0; i < 4; i++) vf[i] = ld16(p.kv.v + pl + (i >> 1) * 2048 + (i & 1) * 512);   // [tile][dims 32 ..]
     if (tid < 32) scl[tid] = (float)((tile_q_scale(p, r0 + min(tid, nr - 1)) * (double)sk) * p.attn_scale);
-    for (int e = tid; e < 32 * 64; e += 256) accs[e] = 0;
-    tile_q_quantize(p, tq, qs8);   // float32 Q quantized while the K and V loads are in flight
+    for (int e = tid; e < 32 * 64; e += NW * 64) accs[e] = 0;
+    if (tid < 256) tile_q_quantize(p, tq, qs8);   // float32 Q quantized while the K and V loads are in flight
     __syncthreads();
     tile_q_frags(p, qs8, col, hi, tq);
-    const v4i qa0 = tq.qa0, qa1 = tq.qa1;
     const float rs = scl[col];
-    const int rpos = pos_first + col;
+    const int rpos = pos_first + col, t0 = 64 * wave + 4 * hi;
+    const bool whole = 64 * wave + 63 <= pos_first;   // every row sees the whole block
 
-    // pass A: scores (kept) and the row maximum
-    float sc[NB][2][16];
-    float mx = -INFINITY;
+    // pass A: scores and each row's largest
+    v16i S[2];
+    int mxs = -2147483647 - 1;
+    if (mine) {
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-        if (wave + 4 * j >= nblk) continue;
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            v16i acc = {};
-            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[j][half][0], qa0, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[j][half][1], qa1, acc, 0, 0, 0);
-            const int t0 = 64 * (wave + 4 * j) + 32 * half + 4 * hi;
-            if (64 * (wave + 4 * j) + 63 <= pos_first) {   // every row sees the whole block
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const float v = (float)acc[i] * rs;
-                    sc[j][half][i] = v;
-                    mx = fmaxf(mx, v);
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const float v = (float)acc[i] * rs;
-                    sc[j][half][i] = v;
-                    const int t = t0 + 8 * (i >> 2) + (i & 3);
-                    mx = t <= rpos ? fmaxf(mx, v) : mx;
-                }
-            }
+        for (int c = 0; c < 2; c++) {
+            S[c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[2 * c], tq.qa0, (v16i){}, 0, 0, 0);
+            S[c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[2 * c + 1], tq.qa1, S[c], 0, 0, 0);
         }
-    }
-    mx = fmaxf(mx, lane_xor<32>(mx));
-    if (hi == 0) wmax[wave][col] = mx;
-    __syncthreads();
-    const float m = fmaxf(fmaxf(wmax[0][col], wmax[1][col]), fmaxf(wmax[2][col], wmax[3][col]));
-
-    // pass B: exponentials (kept) and block sums in the butterfly order
+        if (whole) {
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-        const int b = wave + 4 * j;
-        if (b >= nblk) continue;
-        const int t0 = 64 * b + 4 * hi;
-        // x - m <= 0 for every key a row sees: tl_expf_nonpos is tl_expf there
-        if (64 * b + 63 <= pos_first) {
-#pragma unroll
-            for (int half = 0; half < 2; half++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) sc[j][half][i] = tl_expf_nonpos(sc[j][half][i] - m);
+            for (int i = 0; i < 16; i++) mxs = max(mxs, max(S[0][i], S[1][i]));
         } else {
 #pragma unroll
-            for (int half = 0; half < 2; half++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int t = t0 + 32 * half + 8 * (i >> 2) + (i & 3);
-                    sc[j][half][i] = t <= rpos ? tl_expf_nonpos(sc[j][half][i] - m) : 0.0f;
-                }
+            for (int i = 0; i < 16; i++) {
+                const int t = t0 + 8 * (i >> 2) + (i & 3);
+                mxs = t <= rpos ? max(mxs, S[0][i]) : mxs;
+                mxs = t + 32 <= rpos ? max(mxs, S[1][i]) : mxs;
+            }
         }
-        float a[16];
+        mxs = max(mxs, lane_xor<32>(mxs));
+    }
+    if (hi == 0) wmax[wave][col] = mxs;
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 16; i++) a[i] = sc[j][0][i] + sc[j][1][i];      // distance 32
-        float c[4];
+    for (int w = 0; w < NW; w++) mxs = max(mxs, wmax[w][col]);
+    const float m = (float)mxs * rs;
+
+    // pass B: exponentials (kept) and block sums in the butterfly order
+    float ex[2][16];
+    if (mine) {
+        if (whole) {   // x - m <= 0 for every key a row sees: tl_expf_nonpos is tl_expf there
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float b0 = a[r] + a[r + 8], b1 = a[r + 4] + a[r + 12];      // distance 16
-            c[r] = b0 + b1;                                                   // distance 8
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) ex[c][i] = tl_expf_nonpos((float)S[c][i] * rs - m);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    ex[c][i] = t0 + 32 * c + 8 * (i >> 2) + (i & 3) <= rpos ? tl_expf_nonpos((float)S[c][i] * rs - m) : 0.0f;
         }
         float d[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) d[r] = pair_sum<32>(c[r]);      // distance 4
-        const float f = (d[0] + d[2]) + (d[1] + d[3]);                        // distances 2, 1
-        if (hi == 0) bsum[col * nblk + b] = f;
-    }
-    __syncthreads();
-    if (tid < 32) {
-        const float total = ordered_sum(bsum + tid * nblk, nblk);
-        tot[tid] = total;
+        for (int r = 0; r < 4; r++) {
+            // distance 32 (the two tiles), 16, 8; then 4 across lanes
+            const float b0 = (ex[0][r] + ex[1][r]) + (ex[0][r + 8] + ex[1][r + 8]);
+            const float b1 = (ex[0][r + 4] + ex[1][r + 4]) + (ex[0][r + 12] + ex[1][r + 12]);
+            d[r] = pair_sum<32>(b0 + b1);
+        }
+        const float f = (d[0] + d[2]) + (d[1] + d[3]);   // distances 2, 1
+        if (hi == 0) bsum[col * (NW + 1) + wave] = f;
     }
     __syncthreads();
 
-    // pass C: INT8 probabilities, four consecutive keys per 32-bit store;
+    // pass C: INT8 probabilities and P . V of the wavefront's block;
     // exponential / total correctly rounded from the row's reciprocal and two
     // residual corrections (e <= 1 <= total keeps e y finite; the wave vote
     // confirms every total lies in the quotient's range).  A float sum of
     // nonnegative terms is never below any of them, so 0 <= e <= total and
     // rne(127 e / total) already lies in [0, 127]: the probability clip holds
     // without a clamp, and the byte is packed straight from the float.
-    const float tr = tot[col];
-    const RnDiv dv{tr, __fdiv_rn(1.0f, tr), true};
-    const bool fast = __all(fabsf(tr) >= 0x1p-64f && fabsf(tr) <= 0x1p64f);
+    if (mine) {
+        const float total = ordered_sum(bsum + col * (NW + 1), nblk);
+        const RnDiv dv{total, __fdiv_rn(1.0f, total), true};
+        const bool fast = __all(fabsf(total) >= 0x1p-64f && fabsf(total) <= 0x1p64f);
+        v16i o0 = {}, o1 = {};
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-        const int b = wave + 4 * j;
-        if (b < nblk) {
+        for (int c = 0; c < 2; c++) {
+            unsigned w[4];
 #pragma unroll
-            for (int half = 0; half < 2; half++)
+            for (int q = 0; q < 4; q++) {
+                w[q] = 0;
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    unsigned word = 0;
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const float e = sc[j][half][4 * q + r];
-                        const float pr = __builtin_rintf((fast ? rn_div_fast(e, dv) : __fdiv_rn(e, tr)) * 127.0f);
-                        word = __builtin_amdgcn_cvt_pk_u8_f32(pr, r, word);
-                    }
-                    *(unsigned*)(p8 + col * tpad + 64 * b + 32 * half + 8 * q + 4 * hi) = word;
+                for (int r = 0; r < 4; r++) {
+                    const float e = ex[c][4 * q + r];
+                    const float pr = __builtin_rintf((fast ? rn_div_fast(e, dv) : __fdiv_rn(e, total)) * 127.0f);
+                    w[q] = __builtin_amdgcn_cvt_pk_u8_f32(pr, r, w[q]);
                 }
+            }
+            const v4i pa = prob_frag(w);
+            o0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(pa, vf[2 * c], o0, 0, 0, 0);
+            o1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(pa, vf[2 * c + 1], o1, 0, 0, 0);
         }
-    }
-    __syncthreads();
-
-    // pass D: O = P8 . V
-    v16i o0 = {}, o1 = {};
 #pragma unroll
-    for (int j = 0; j < 2 * NB; j++) {
-        const int kc = wave + 4 * j;
-        if (kc < tpad / 32) {
-            const v4i a = *(const v4i*)(p8 + col * tpad + kc * 32 + hi * 16);
-            o0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, vf[j][0], o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, vf[j][1], o1, 0, 0, 0);
+        for (int i = 0; i < 16; i++) {
+            const int r = 8 * (i >> 2) + 4 * hi + (i & 3);
+            atomicAdd(&accs[r * 64 + col], o0[i]);
+            atomicAdd(&accs[r * 64 + 32 + col], o1[i]);
         }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int r = 8 * (i >> 2) + 4 * hi + (i & 3);
-        atomicAdd(&accs[r * 64 + col], o0[i]);
-        atomicAdd(&accs[r * 64 + 32 + col], o1[i]);
     }
     __syncthreads();
     const float pv_mult = deq_mult(1.0 / 127.0, sv);
-    for (int e = tid; e < 32 * 64; e += 256) {
+    for (int e = tid; e < 32 * 64; e += NW * 64) {
         const int r = e >> 6, d = e & 63;
         if (r < nr) p.out[(int64_t)(r0 + r) * D + (int64_t)h * kHeadDim + d] = (float)accs[e] * pv_mult;
     }
@@ -2292,13 +2268,26 @@ hipError_t launch_attention_tiles(hipStream_t s, const int8_t* q8, const double*
         (qf && !qmax) || (!qf && (!q8 || !q_scale)))
         return hipErrorInvalidValue;
     const int tpad = (pos0 + rows + 63) & ~63;
-    const size_t lds = tile_lds_bytes(tpad);
     AttnTileArgs a{q8, q_scale, n_heads, n_kv_heads, rows, seq, pos0, layer, kv, kv_sk, kv_sv,
                    1.0 / sqrt((double)kHeadDim), out, qf, qmax};
     const dim3 grid(n_heads, (rows + 31) / 32), block(256);
-    if (tpad <= 256) TL_KLAUNCH(attention_tile_reg_kernel<1>, grid, block, lds, s, a);
-    else if (tpad <= 512) TL_KLAUNCH(attention_tile_reg_kernel<2>, grid, block, lds, s, a);
-    else TL_KLAUNCH(attention_tile_kernel, grid, block, lds, s, a);
+    // Wavefronts per tile: one 64-key block each while the context allows
+    // (up to 512 keys; up to 1024 while one round of 16-wavefront workgroups
+    // covers the tiles: 13.2 us against 18-19 at 60-124 rows behind 900 keys).
+    // Longer contexts: more wavefronts shorten a tile's serial walk over the
+    // keys but hold fewer tiles per CU, so the count follows the number of
+    // tiles: 16 up to one per CU (100 rows behind 1500 keys: 20.3 us against 23.2
+    // with 8), 8 below four per CU (512 rows behind 512 keys: 24.2 against
+    // 28.7 with 4), else 4 (1024 rows from key 0: 31.2 against 35.7; 2048:
+    // 74.0 against 81.8).
+    const int wgs = n_heads * (int)grid.y;
+    const size_t lds = tile_lds_bytes(tpad / 64);
+    if (tpad <= 256) TL_KLAUNCH(attention_tile_reg_kernel<4>, grid, block, 0, s, a);
+    else if (tpad <= 512) TL_KLAUNCH(attention_tile_reg_kernel<8>, grid, dim3(512), 0, s, a);
+    else if (tpad <= 1024 && wgs <= 256) TL_KLAUNCH(attention_tile_reg_kernel<16>, grid, dim3(1024), 0, s, a);
+    else if (wgs <= 256) TL_KLAUNCH(attention_tile_kernel<16>, grid, dim3(1024), lds, s, a);
+    else if (wgs < 1024) TL_KLAUNCH(attention_tile_kernel<8>, grid, dim3(512), lds, s, a);
+    else TL_KLAUNCH(attention_tile_kernel<4>, grid, block, lds, s, a);
     return hipGetLastError();
 }
 

@@ -1134,7 +1134,6 @@ int32_t tl_create(const tl_config* cfg, int32_t max_seqs, tl_handle** out) {
     }
     if ((e = init_kernels())) return bad(e);
     if ((e = init_decode_kernels())) return bad(e);
-    if ((e = init_prefill_kernels())) return bad(e);
     if ((e = init_gemm_pk_kernels())) return bad(e);
     if ((e = init_skinny_kernels())) return bad(e);
     if (const char* env = std::getenv("TL_BATCH_O_FUSE")) h->o_fuse = env[0] != '0';
