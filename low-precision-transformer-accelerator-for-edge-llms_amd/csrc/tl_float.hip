@@ -13,67 +13,141 @@ namespace tl {
 
 namespace {
 
-constexpr int kLB = 64;   // output tile 64 x 64, one 4 x 4 block per thread
-constexpr int kLK = 16;   // K step staged through LDS
+typedef float v16f __attribute__((ext_vector_type(16)));
 
-__global__ __launch_bounds__(256) void linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                         const float* __restrict__ b,
-                                                         const float* __restrict__ residual, int32_t m, int32_t n,
-                                                         int32_t k, float* __restrict__ y) {
-    __shared__ float as[kLK][kLB + 4];   // [k][row]
-    __shared__ float bs[kLK][kLB];       // [k][col]
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int row0 = blockIdx.y * kLB, col0 = blockIdx.x * kLB;
-    float acc[4][4];
+// y = x . W on v_mfma_f32_32x32x2_f32 (one multiply-add per product, float32
+// accumulators): a workgroup of 8 wavefronts per 32 x (32 NB) output tile, each
+// over an eighth of K, partial tiles added in LDS in a fixed order.  In a chunk
+// of 8 k's lane l holds x[row l % 32][4 (l / 32) .. + 3] (one 16-byte load) and
+// multiplies k = s and k = 4 + s in step s, so its W operand is row
+// 4 (l / 32) + s, column l % 32 of each column block: 128-byte runs of W
+// straight into registers, no LDS and no barrier in the main loop.
+// What bounds it: the float32 matrix rate at hundreds of rows (640 x 5632 x
+// 2048: 90 TFLOP/s; 100 x 5632 x 2048 puts 236 of 256 CUs at work), launch and
+// latency at a few.  The whole call at 100 x 5632 x 2048: 245 us with 64 x 64 vector-FMA
+// tiles through LDS, 53 us now; 640 rows 407 -> 175; one row 238 -> 30.  Eight
+// partial sums per output also round less: 2.9e-7 relative to 64 bits where
+// one chain of 2048 had 8.1e-7.
+constexpr int kLinWaves = 8;
+
+template <int NB, bool VEC>
+__global__ __launch_bounds__(kLinWaves * 64) void linear_f32_kernel(const float* __restrict__ x,
+                                                                    const float* __restrict__ w,
+                                                                    const float* __restrict__ b,
+                                                                    const float* __restrict__ residual, int32_t m,
+                                                                    int32_t n, int32_t k, int32_t tiles_m,
+                                                                    int32_t tiles_n, float* __restrict__ y) {
+    constexpr int PD = NB == 1 ? 8 : 4, HW = kLinWaves / 2;   // chunks in flight; LDS partial tiles
+    __shared__ float red[HW][NB * 16][64];
+    // workgroups go to the 8 XCDs round-robin: the row tiles of a column tile
+    // stay on one XCD, whose L2 then holds the column tile's weights
+    const int q = (int)blockIdx.x >> 3, tn = q / tiles_m * 8 + ((int)blockIdx.x & 7), tm = q % tiles_m;
+    if (tn >= tiles_n) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), col = lane & 31, hi = lane >> 5;
+    const int64_t row0 = (int64_t)tm * 32;
+    const int col0 = tn * 32 * NB;
+    const int nfull = k >> 3, nch = (k + 7) >> 3, per = (nch + kLinWaves - 1) / kLinWaves;
+    const int c0 = min(wave * per, nfull), c1 = min(c0 + per, nfull);   // this wavefront's whole chunks
+    // one wavefront-uniform base per chunk and 32-bit lane offsets: no 64-bit
+    // address arithmetic per load
+    const float* xb = x + row0 * k;
+    const unsigned xo = (unsigned)min(col, (int)(m - 1 - row0)) * (unsigned)k + 4 * hi;
+    unsigned wo[4][NB];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int s = 0; s < 4; s++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = 0.0f;
-    const int ar = tid >> 2, ak = (tid & 3) * 4;    // A: row ar, k ak..ak+3
-    const int bk = tid >> 4, bc = (tid & 15) * 4;   // B: k bk, cols bc..bc+3
-    for (int k0 = 0; k0 < k; k0 += kLK) {
-        const int gr = row0 + ar;
+        for (int j = 0; j < NB; j++) wo[s][j] = (unsigned)(4 * hi + s) * (unsigned)n + (unsigned)min(col0 + 32 * j + col, n - 1);
+    v16f acc[NB];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int gk = k0 + ak + j;
-            as[ak + j][ar] = (gr < m && gk < k) ? x[(int64_t)gr * k + gk] : 0.0f;
+    for (int j = 0; j < NB; j++) acc[j] = (v16f){};
+    float av[PD][4], bv[PD][4][NB];
+    auto load = [&](int set, int c) {
+        const float* xc = xb + 8 * (int64_t)c;
+        const float* wc = w + 8 * (int64_t)c * n;
+        if constexpr (VEC) {
+            const float4 v = *(const float4*)(xc + xo);
+            av[set][0] = v.x; av[set][1] = v.y; av[set][2] = v.z; av[set][3] = v.w;
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; s++) av[set][s] = xc[xo + s];
         }
-        const int gk = k0 + bk;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int gc = col0 + bc + j;
-            bs[bk][bc + j] = (gk < k && gc < n) ? w[(int64_t)gk * n + gc] : 0.0f;
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int j = 0; j < NB; j++) bv[set][s][j] = wc[wo[s][j]];
+    };
+    auto mma = [&](int set) {
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[set][s], bv[set][s][j], acc[j], 0, 0, 0);
+    };
+    if (c0 < c1) {
+#pragma unroll
+        for (int u = 0; u < PD; u++) load(u, min(c0 + u, c1 - 1));
+        int c = c0;
+        for (; c + PD <= c1; c += PD) {
+#pragma unroll
+            for (int u = 0; u < PD; u++) {
+                mma(u);
+                load(u, min(c + u + PD, c1 - 1));   // past the end: a redundant load in bounds
+                __builtin_amdgcn_sched_barrier(0);  // the loads stay here: PD - 1 chunks of MFMAs cover them
+            }
         }
-        __syncthreads();
 #pragma unroll
-        for (int kk = 0; kk < kLK; kk++) {
-            float a[4], bb[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) a[i] = as[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; j++) bb[j] = bs[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = __builtin_fmaf(a[i], bb[j], acc[i][j]);
-        }
-        __syncthreads();
+        for (int u = 0; u < PD - 1; u++)
+            if (c + u < c1) mma(u);
     }
+    if (nch > nfull && wave == kLinWaves - 1) {   // the last k % 8: zeros past k on both sides
+        const int64_t kk = 8 * (int64_t)nfull + 4 * hi;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int r = row0 + ty * 4 + i;
-        if (r >= m) continue;
+        for (int s = 0; s < 4; s++) {
+            const bool in = kk + s < k;
+            av[0][s] = in ? xb[8 * (int64_t)nfull + xo + s] : 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int c = col0 + tx * 4 + j;
-            if (c >= n) continue;
-            float v = acc[i][j];
-            if (b) v = v + b[c];
-            const int64_t idx = (int64_t)r * n + c;
-            if (residual) v = residual[idx] + v;
-            y[idx] = v;
+            for (int j = 0; j < NB; j++) bv[0][s][j] = in ? w[8 * (int64_t)nfull * n + wo[s][j]] : 0.0f;
         }
+        mma(0);
     }
+    // wavefront h + 4's tile into LDS, wavefront h adds its own, then every
+    // thread adds four partial sums per output in wavefront order
+    if (wave >= HW) {
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) red[wave - HW][j * 16 + e][lane] = acc[j][e];
+    }
+    __syncthreads();
+    if (wave < HW) {
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) red[wave][j * 16 + e][lane] = acc[j][e] + red[wave][j * 16 + e][lane];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2 * NB; i++) {   // output register e of block j: 16 NB of them over 8 wavefronts
+        const int je = i * kLinWaves + wave, e = je & 15;
+        const int64_t r = row0 + 8 * (e >> 2) + 4 * hi + (e & 3);
+        const int c = col0 + 32 * (je >> 4) + col;
+        if (r >= m || c >= n) continue;
+        float v = (red[0][je][lane] + red[1][je][lane]) + (red[2][je][lane] + red[3][je][lane]);
+        if (b) v = v + b[c];
+        const int64_t idx = r * n + c;
+        if (residual) v = residual[idx] + v;
+        y[idx] = v;
+    }
+}
+
+template <int NB>
+void go_linear(hipStream_t s, const float* x, const float* w, const float* b, const float* residual, int32_t m,
+               int32_t n, int32_t k, float* y) {
+    const int32_t tm = (int32_t)(((int64_t)m + 31) / 32), tn = (n + 32 * NB - 1) / (32 * NB);
+    const dim3 grid((unsigned)((tn + 7) / 8 * 8) * (unsigned)tm), block(kLinWaves * 64);
+    if (k % 4 == 0 && (uintptr_t)x % 16 == 0)
+        TL_KLAUNCH((linear_f32_kernel<NB, true>), grid, block, 0, s, x, w, b, residual, m, n, k, tm, tn, y);
+    else TL_KLAUNCH((linear_f32_kernel<NB, false>), grid, block, 0, s, x, w, b, residual, m, n, k, tm, tn, y);
 }
 
 // one (query row i, query head h) per workgroup; the row's scores live in LDS
@@ -148,8 +222,24 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
 hipError_t launch_linear_f32(hipStream_t s, const float* x, const float* w, const float* b, const float* residual,
                              int32_t m, int32_t n, int32_t k, float* y) {
     if (m <= 0 || n <= 0) return hipSuccess;
-    const dim3 grid((n + kLB - 1) / kLB, (m + kLB - 1) / kLB);
-    TL_KLAUNCH(linear_f32_kernel, grid, dim3(256), 0, s, x, w, b, residual, m, n, k, y);
+    // column blocks per tile: the fewest MFMAs on the busiest CU (rounds of 256
+    // tiles times blocks); of equals the widest, which reads x least often
+    const int64_t tm = ((int64_t)m + 31) / 32;
+    int nb = 1;
+    int64_t best = INT64_MAX;
+    for (int c = 1; c <= 4; c++) {
+        const int64_t cost = (tm * (((int64_t)n + 32 * c - 1) / (32 * c)) + 255) / 256 * c;
+        if (cost <= best) {
+            best = cost;
+            nb = c;
+        }
+    }
+    switch (nb) {
+        case 1: go_linear<1>(s, x, w, b, residual, m, n, k, y); break;
+        case 2: go_linear<2>(s, x, w, b, residual, m, n, k, y); break;
+        case 3: go_linear<3>(s, x, w, b, residual, m, n, k, y); break;
+        default: go_linear<4>(s, x, w, b, residual, m, n, k, y); break;
+    }
     return hipGetLastError();
 }
 
