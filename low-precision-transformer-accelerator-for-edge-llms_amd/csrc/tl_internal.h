@@ -322,8 +322,22 @@ hipError_t launch_attention_decode(hipStream_t s, const float* qkv, int32_t rows
 hipError_t launch_embed_step(hipStream_t s, const int32_t* tok_by_seq, const int32_t* seq_of_row, int32_t rows,
                              const int32_t* cursor, int32_t* row_pos, int32_t d, int32_t vocab, const int8_t* emb,
                              const float* emb_s, float* x);
-hipError_t launch_step_rows(hipStream_t s, const int32_t* seq_of_row, int32_t rows,
-                            const int32_t* cursor, int32_t* row_pos);
+// the sequence and position of rows 0 .. rows - 1 (one sequence, or row r is
+// sequence seq + r with per_row), and the state of one sequence where the
+// pointers are given.  The values travel as kernel arguments: no copy from host
+// memory and no wait for one.
+struct RowsInit {
+    int32_t* row_seq;
+    int32_t* row_pos;
+    int32_t rows, seq, pos0, per_row;
+    int32_t* n_gen;             // = 0
+    int32_t* cursor;            // = cursor_v
+    unsigned long long* key;    // = 0
+    int32_t* eos;               // = eos_v (< 0: none)
+    int32_t* stopped;           // = 0
+    int32_t cursor_v, eos_v;
+};
+hipError_t launch_rows_init(hipStream_t s, const RowsInit& a);
 hipError_t launch_kv_scatter(hipStream_t s, KvGeom kv, int32_t seq, int32_t layer, int32_t g,
                              int32_t t0, int32_t n, const int8_t* k_rows, const int8_t* v_rows);
 hipError_t launch_kv_gather(hipStream_t s, KvGeom kv, int32_t seq, int32_t layer, int32_t g,

@@ -1617,13 +1617,20 @@ hipError_t launch_argmax_tiles(hipStream_t s, const unsigned long long* part, in
 }
 
 // batched decode: the position of each row is its sequence's cursor
-__global__ void step_rows_kernel(const int32_t* seq_of_row, int32_t rows, const int32_t* cursor,
-                                 int32_t* row_pos) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < rows) row_pos[r] = cursor[seq_of_row[r]];
+__global__ __launch_bounds__(256) void rows_init_kernel(RowsInit a) {
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r < a.rows) {
+        a.row_seq[r] = a.per_row ? a.seq + r : a.seq;
+        a.row_pos[r] = a.pos0 + r;
+    }
+    if (r != 0) return;
+    if (a.n_gen) *a.n_gen = 0;
+    if (a.cursor) *a.cursor = a.cursor_v;
+    if (a.key) *a.key = 0ull;
+    if (a.eos) *a.eos = a.eos_v;
+    if (a.stopped) *a.stopped = 0;
 }
 
-// logical [n][64] rows <-> cache plane layout
 __global__ void kv_scatter_kernel(KvGeom kv, int64_t pl, int32_t t0, int32_t n,
                                   const int8_t* __restrict__ k_rows, const int8_t* __restrict__ v_rows) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2377,10 +2384,8 @@ hipError_t init_kernels() {
                                150 * 1024);
 }
 
-hipError_t launch_step_rows(hipStream_t s, const int32_t* seq_of_row, int32_t rows,
-                            const int32_t* cursor, int32_t* row_pos) {
-    TL_KLAUNCH(step_rows_kernel, dim3(ceil_div(rows, 64)), dim3(64), 0, s, seq_of_row, rows,
-                       cursor, row_pos);
+hipError_t launch_rows_init(hipStream_t s, const RowsInit& a) {
+    TL_KLAUNCH(rows_init_kernel, dim3(std::max(1, ceil_div(a.rows, 256))), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -168,12 +168,15 @@ struct tl_handle {
     int32_t* tokens_out = nullptr;   // [max_seqs][max_pos]
     float* logit_out = nullptr;      // [max_seqs][max_pos]
     std::vector<int32_t> host_cursor;
-    int32_t stop_state[2] = {-1, 0};  // host words copied into eos_id / stopped
     // pinned host words the device reads and writes: [0] the abort word the
     // token bookkeeping kernel checks every step, [1 + seq] the mirror of
     // stopped[seq] it writes (1 EOS, 2 host abort)
     int32_t* ctl_host = nullptr;      // host view
     int32_t* ctl_dev = nullptr;       // device view of the same words
+    // pinned host words: argmax keys of the LM-head operator's workgroups,
+    // written by the kernel, folded by the host
+    unsigned long long* wg_keys_host = nullptr;   // host view, [vocab / 4]
+    unsigned long long* wg_keys_dev = nullptr;    // device view of the same words
     hipEvent_t watch_ev[kWatchDepth] = {};
     std::vector<int32_t> host_ngen;
 
@@ -871,32 +874,50 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
     return TL_OK;
 }
 
-int32_t upload_rows(tl_handle* h, int32_t rows, int32_t seq_first, bool seq_per_row, int32_t pos0) {
-    std::vector<int32_t> s(rows), p(rows);
-    for (int i = 0; i < rows; i++) {
-        s[i] = seq_per_row ? seq_first + i : seq_first;
-        p[i] = pos0 + i;
-    }
+// rows 0 .. rows - 1 of the workspaces: their sequences and positions
+RowsInit rows_init(tl_handle* h, int32_t rows, int32_t seq_first, bool seq_per_row, int32_t pos0) {
     h->rows_one_seq = !seq_per_row;
     h->rows_seq = seq_first;
     h->rows_pos0 = pos0;
-    TL_HIP(h, hipMemcpyAsync(h->row_seq, s.data(), rows * sizeof(int32_t), hipMemcpyHostToDevice, h->stream));
-    TL_HIP(h, hipMemcpyAsync(h->row_pos, p.data(), rows * sizeof(int32_t), hipMemcpyHostToDevice, h->stream));
-    // the host vectors must outlive the async copies
-    TL_HIP(h, hipStreamSynchronize(h->stream));
+    RowsInit a{};
+    a.row_seq = h->row_seq; a.row_pos = h->row_pos;
+    a.rows = rows; a.seq = seq_first; a.pos0 = pos0; a.per_row = seq_per_row;
+    return a;
+}
+
+int32_t set_rows(tl_handle* h, int32_t rows, int32_t seq_first, bool seq_per_row, int32_t pos0) {
+    TL_LAUNCH(h, launch_rows_init(h->stream, rows_init(h, rows, seq_first, seq_per_row, pos0)));
     return TL_OK;
 }
 
-// the EOS id a sequence's decode steps check, and its stop flag cleared
-int32_t set_stop_state(tl_handle* h, int32_t seq, int32_t eos_id) {
-    h->stop_state[0] = eos_id < 0 ? -1 : eos_id;
-    h->stop_state[1] = 0;
-    TL_HIP(h, hipMemcpyAsync(h->eos_id + seq, &h->stop_state[0], sizeof(int32_t), hipMemcpyHostToDevice, h->stream));
-    TL_HIP(h, hipMemcpyAsync(h->stopped + seq, &h->stop_state[1], sizeof(int32_t), hipMemcpyHostToDevice, h->stream));
-    // the host words must stay unchanged until the copies have run
-    TL_HIP(h, hipStreamSynchronize(h->stream));
+// row 0 of the workspaces for decode steps of sequence seq at position pos,
+// with the EOS id the steps check and the stop flag cleared
+int32_t set_decode_row(tl_handle* h, int32_t seq, int32_t pos, int32_t eos_id) {
+    RowsInit a = rows_init(h, 1, seq, false, pos);
+    a.eos = h->eos_id + seq; a.eos_v = eos_id < 0 ? -1 : eos_id;
+    a.stopped = h->stopped + seq;
+    TL_LAUNCH(h, launch_rows_init(h->stream, a));
     return TL_OK;
 }
+
+// The single-layer entry points run on the caller's rows in place: the layer's
+// kernels read and write h->x, which is the caller's buffer while this lives.
+// The kernels use 16-byte accesses; an unaligned buffer is copied in and out
+// instead (copy()).
+struct CallerRows {
+    tl_handle* h;
+    float* own;
+    float* x;
+    size_t bytes;
+    bool copy;
+    CallerRows(tl_handle* hh, float* xx, int32_t rows)
+        : h(hh), own(hh->x), x(xx), bytes(sizeof(float) * (size_t)hh->D * rows), copy((uintptr_t)xx % 16 != 0) {
+        if (!copy) h->x = x;
+    }
+    ~CallerRows() { h->x = own; }
+    hipError_t in() const { return copy ? hipMemcpyAsync(own, x, bytes, hipMemcpyDeviceToDevice, h->stream) : hipSuccess; }
+    hipError_t out() const { return copy ? hipMemcpyAsync(x, own, bytes, hipMemcpyDeviceToDevice, h->stream) : hipSuccess; }
+};
 
 // clears the abort word when a watched decode or prefill returns (also on an
 // error path), so no later step of another call reads a stale abort
@@ -1129,6 +1150,12 @@ int32_t tl_create(const tl_config* cfg, int32_t max_seqs, tl_handle** out) {
         std::memset(hp, 0, sizeof(int32_t) * words);
         if ((e = hipHostGetDevicePointer(&dp, hp, 0))) return bad(e);
         h->ctl_dev = (int32_t*)dp;
+        if ((e = hipHostMalloc(&hp, sizeof(unsigned long long) * (size_t)((c.vocab + 3) / 4),
+                               hipHostMallocMapped | hipHostMallocCoherent)))
+            return bad(e);
+        h->wg_keys_host = (unsigned long long*)hp;
+        if ((e = hipHostGetDevicePointer(&dp, hp, 0))) return bad(e);
+        h->wg_keys_dev = (unsigned long long*)dp;
         for (auto& ev : h->watch_ev)
             if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming))) return bad(e);
     }
@@ -1160,6 +1187,7 @@ void tl_destroy(tl_handle* h) {
     for (auto e : h->watch_ev)
         if (e) (void)hipEventDestroy(e);
     if (h->ctl_host) (void)hipHostFree(h->ctl_host);
+    if (h->wg_keys_host) (void)hipHostFree(h->wg_keys_host);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
 }
@@ -1492,7 +1520,7 @@ int32_t tl_qkv_append(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, in
     TL_REQ(h, rows >= 1 && rows <= h->max_rows && pos0 >= 0 && (int64_t)pos0 + rows <= c.max_pos,
            "position range out of bounds");
     TL_REQ(h, qkv && q8 && q_scale, "null pointer");
-    int32_t r = upload_rows(h, rows, seq, false, pos0);
+    int32_t r = set_rows(h, rows, seq, false, pos0);
     if (r) return r;
     TL_LAUNCH(h, launch_qkv_post(h->stream, qkv, rows, c.n_heads, c.n_kv_heads, rowmap(h), h->rope_cos, h->rope_sin,
                                  h->kv, layer, h->kv_sk, h->kv_sv, q8, q_scale, q_rot));
@@ -1507,7 +1535,7 @@ int32_t tl_attention(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, int
     TL_REQ(h, rows >= 1 && rows <= h->max_rows && pos0 >= 0 && (int64_t)pos0 + rows <= c.max_pos,
            "position range out of bounds");
     TL_REQ(h, q8 && q_scale && out, "null pointer");
-    int32_t r = upload_rows(h, rows, seq, false, pos0);
+    int32_t r = set_rows(h, rows, seq, false, pos0);
     if (r) return r;
     {
         Prof p(h, TL_K_ATTN, 0.0);
@@ -1520,21 +1548,43 @@ int32_t tl_lm_head_argmax(tl_handle* h, const float* x, int32_t* token, float* l
     if (!h) return TL_ERR_BAD_DESCRIPTOR;
     TL_REQ(h, x && token, "null pointer");
     const int D = h->D, V = h->cfg.vocab;
-    TL_LAUNCH(h, launch_reset_keys(h->stream, h->op_key, 1));
-    {
-        Prof p(h, TL_K_NORM, D * 9.0);
-        TL_LAUNCH(h, launch_rmsnorm_quant(h->stream, x, h->g_final, 1, D, h->cfg.rms_eps, h->plan, nullptr, h->a8, h->as));
-    }
-    GemvArgs g{};
-    g.w = h->lm_w; g.ws = h->lm_s; g.x = h->a8; g.xs = h->as; g.key = h->op_key; g.y = logits; g.n = V; g.k = D;
-    {
-        Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + D);
-        TL_LAUNCH(h, launch_gemv(h->stream, EPI_ARGMAX, g));
-    }
     unsigned long long key = 0;
-    TL_HIP(h, hipMemcpyAsync(&key, h->op_key, sizeof key, hipMemcpyDeviceToHost, h->stream));
-    int32_t r = finish(h);
-    if (r) return r;
+    const int32_t n_wg = gemv_fused_workgroups(PRO_RMSNORM, EPI_ARGMAX, V, D);
+    if ((uintptr_t)x % 16 == 0 && n_wg > 0 && n_wg <= (V + 3) / 4) {
+        // the decode step's fused RMSNorm + LM head; its workgroups store their
+        // best keys straight into pinned host memory, which is folded here once the
+        // kernel has ended (57 -> 31 us per call against a norm kernel, a GEMV with one
+        // atomicMax per workgroup and a copy of the key)
+        GemvArgs g = gemv_args(h);
+        g.xf = x; g.gamma = h->g_final; g.w = h->lm_w; g.ws = h->lm_s; g.y = logits; g.n = V; g.k = D;
+        g.key = h->op_key;
+        g.wg_keys = h->wg_keys_dev;
+        {
+            Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + D * 8.0);
+            TL_LAUNCH(h, launch_gemv_fused(h->stream, PRO_RMSNORM, EPI_ARGMAX, g));
+        }
+        const int32_t r = finish(h);
+        if (r) return r;
+        for (int32_t i = 0; i < n_wg; i++) {
+            const unsigned long long k = ((volatile unsigned long long*)h->wg_keys_host)[i];
+            key = std::max(key, k);
+        }
+    } else {   // rows off 16 bytes: the row kernel that takes them, then the GEMV
+        TL_LAUNCH(h, launch_reset_keys(h->stream, h->op_key, 1));
+        {
+            Prof p(h, TL_K_NORM, D * 9.0);
+            TL_LAUNCH(h, launch_rmsnorm_quant(h->stream, x, h->g_final, 1, D, h->cfg.rms_eps, h->plan, nullptr, h->a8, h->as));
+        }
+        GemvArgs g{};
+        g.w = h->lm_w; g.ws = h->lm_s; g.x = h->a8; g.xs = h->as; g.key = h->op_key; g.y = logits; g.n = V; g.k = D;
+        {
+            Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + D);
+            TL_LAUNCH(h, launch_gemv(h->stream, EPI_ARGMAX, g));
+        }
+        TL_HIP(h, hipMemcpyAsync(&key, h->op_key, sizeof key, hipMemcpyDeviceToHost, h->stream));
+        const int32_t r = finish(h);
+        if (r) return r;
+    }
     *token = (int32_t)(0xFFFFFFFFu - (unsigned)(key & 0xFFFFFFFFull));
     if (logit) {
         unsigned u = (unsigned)(key >> 32);
@@ -1560,11 +1610,12 @@ int32_t tl_decode_layer(tl_handle* h, int32_t seq, int32_t layer, int32_t pos, f
     TL_REQ(h, pos >= 0 && pos < c.max_pos, "position out of range");
     TL_REQ(h, x, "null pointer");
     if (!h->layers[layer].wqkv) return fail(h, TL_ERR_BAD_DESCRIPTOR, "layer not loaded");
-    int32_t r = upload_rows(h, 1, seq, false, pos);
+    int32_t r = set_rows(h, 1, seq, false, pos);
     if (r) return r;
-    TL_HIP(h, hipMemcpyAsync(h->x, x, sizeof(float) * h->D, hipMemcpyDeviceToDevice, h->stream));
+    const CallerRows cx(h, x, 1);
+    TL_HIP(h, cx.in());
     if ((r = layer_rows(h, layer, 1, pos + 1, true))) return r;
-    TL_HIP(h, hipMemcpyAsync(x, h->x, sizeof(float) * h->D, hipMemcpyDeviceToDevice, h->stream));
+    TL_HIP(h, cx.out());
     return finish(h);
 }
 
@@ -1588,13 +1639,13 @@ int32_t prefill_layers(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t
     if (r) return r;
     h->host_ngen[seq] = 0;   // the sequence is rewritten: no decode until prefill_finish
     h->host_cursor[seq] = 0;
-    if ((r = upload_rows(h, n, seq, false, 0))) return r;
     TL_HIP(h, hipMemcpyAsync(h->tokens, tokens, sizeof(int32_t) * n, hipMemcpyHostToDevice, h->stream));
-    const int32_t zero = 0;
-    TL_HIP(h, hipMemcpyAsync(h->n_gen + seq, &zero, sizeof zero, hipMemcpyHostToDevice, h->stream));
-    TL_HIP(h, hipMemcpyAsync(h->cursor + seq, &n, sizeof n, hipMemcpyHostToDevice, h->stream));
-    TL_LAUNCH(h, launch_reset_keys(h->stream, h->keys + seq, 1));
-    if ((r = set_stop_state(h, seq, -1))) return r;
+    RowsInit init = rows_init(h, n, seq, false, 0);
+    init.n_gen = h->n_gen + seq; init.cursor = h->cursor + seq; init.cursor_v = n;
+    init.key = h->keys + seq;
+    init.eos = h->eos_id + seq; init.eos_v = -1;
+    init.stopped = h->stopped + seq;
+    TL_LAUNCH(h, launch_rows_init(h->stream, init));
     TL_LAUNCH(h, launch_embed(h->stream, h->tokens, n, h->D, h->cfg.vocab, h->emb, h->emb_s, h->x));
     for (int l = 0; l < c.n_layers; l++) {
         if (abort_flag) {
@@ -1666,11 +1717,12 @@ int32_t tl_layer_rows(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, in
     TL_REQ(h, pos0 >= 0 && (int64_t)pos0 + rows <= c.max_pos, "Sequence length exceeds max_position_embeddings");
     TL_REQ(h, x, "null pointer");
     if (!h->layers[layer].wqkv) return fail(h, TL_ERR_BAD_DESCRIPTOR, "layer not loaded");
-    int32_t r = upload_rows(h, rows, seq, false, pos0);
+    int32_t r = set_rows(h, rows, seq, false, pos0);
     if (r) return r;
-    TL_HIP(h, hipMemcpyAsync(h->x, x, sizeof(float) * h->D * rows, hipMemcpyDeviceToDevice, h->stream));
+    const CallerRows cx(h, x, rows);
+    TL_HIP(h, cx.in());
     if ((r = layer_rows(h, layer, rows, pos0 + rows, rows == 1))) return r;
-    TL_HIP(h, hipMemcpyAsync(x, h->x, sizeof(float) * h->D * rows, hipMemcpyDeviceToDevice, h->stream));
+    TL_HIP(h, cx.out());
     return finish(h);
 }
 
@@ -1696,8 +1748,7 @@ int32_t tl_decode(tl_handle* h, int32_t seq, int32_t max_new, int32_t eos_id, co
     if (stop_reason) *stop_reason = TL_STOP_NONE;
     const int32_t first = h->host_ngen[seq];
     int32_t r;
-    if ((r = set_stop_state(h, seq, eos_id))) return r;
-    if ((r = upload_rows(h, 1, seq, false, h->host_cursor[seq]))) return r;
+    if ((r = set_decode_row(h, seq, h->host_cursor[seq], eos_id))) return r;
     if ((r = decode_embed1(h))) return r;
     auto launch_step = [&](int32_t i) -> int32_t {
         if (!h->profiling) return decode_graph_launch(h, seq);
@@ -1821,7 +1872,7 @@ int32_t tl_decode_batch(tl_handle* h, int32_t n_seqs, const int32_t* tokens, con
     }
     int32_t r = check_model_loaded(h);
     if (r) return r;
-    if ((r = upload_rows(h, n_seqs, 0, true, 0))) return r;
+    if ((r = set_rows(h, n_seqs, 0, true, 0))) return r;
     std::vector<int32_t> zeros(n_seqs, 0);
     TL_HIP(h, hipMemcpyAsync(h->token_cur, tokens, sizeof(int32_t) * n_seqs, hipMemcpyHostToDevice, h->stream));
     TL_HIP(h, hipMemcpyAsync(h->cursor, start_pos, sizeof(int32_t) * n_seqs, hipMemcpyHostToDevice, h->stream));
@@ -1944,13 +1995,12 @@ int32_t tl_capture_step(tl_handle* h, int32_t seq, tl_capture* cap) {
     TL_REQ(h, cap->n_keys >= 0 && (int64_t)cap->key0 + cap->n_keys <= pos + 1, "attention window outside keys 0..pos");
     int32_t r = check_model_loaded(h);
     if (r) return r;
-    if ((r = set_stop_state(h, seq, -1))) return r;
     const int D = h->D, V = c.vocab;
     const int32_t first = h->host_ngen[seq];
     CaptureScratch sc(h->stream);
     float* xin = sc.get<float>(D);
     if (!xin) return fail(h, TL_ERR_INTERNAL, "hipMalloc");
-    if ((r = upload_rows(h, 1, seq, false, pos))) return r;
+    if ((r = set_decode_row(h, seq, pos, -1))) return r;
     cap->pos = pos;
     TL_HIP(h, hipMemcpyAsync(&cap->token_in, h->token_cur + seq, sizeof(int32_t), hipMemcpyDeviceToHost, h->stream));
     // one step of decode_step1, eagerly
@@ -2037,8 +2087,7 @@ int32_t tl_decode_timeline(tl_handle* h, int32_t seq, int32_t n_steps, tl_timeli
         h->ts_cap = (size_t)1 << 22;
         TL_HIP(h, dalloc(h, &h->ts_buf, h->ts_cap));
     }
-    if ((r = set_stop_state(h, seq, -1))) return r;
-    if ((r = upload_rows(h, 1, seq, false, h->host_cursor[seq]))) return r;
+    if ((r = set_decode_row(h, seq, h->host_cursor[seq], -1))) return r;
     if ((r = decode_embed1(h))) return r;
     // capture one step with stamp regions
     h->ts_on = true;
