@@ -820,6 +820,13 @@ __global__ __launch_bounds__(256) void gemm_pk_split_kernel(GemmArgs a, QkvRopeA
         for (int e = 0; e < 16; e++) {
             const int m = rb + 8 * (e >> 2) + (e & 3);
             const float v = (float)sum[e] * deq_mult(so.sx[bw][e], so.sw[bw]);
+            if constexpr (EPI == EPI_ARGMAX) {
+                // the best key of row m over the block's 32 columns (the
+                // lanes of a half-wavefront), as gemm_rows32_kernel's
+                const unsigned long long k = half_max_u64(argmax_key(v, n));
+                if ((lane & 31) == 0 && m < a.m) a.key[(int64_t)(nt0 + j) * a.m + m] = k;
+                continue;
+            }
             if (m < a.m) a.y[(int64_t)m * a.n + n] = RES ? so.res[bw][RES ? e : 0] + v : v;
         }
     }
@@ -988,6 +995,7 @@ static bool pk_split_narrow(int32_t m, int32_t n) {
 bool gemm_pk_supported(int epi, int32_t m, int32_t n, int32_t k) {
     if (m < 1 || n < 1 || k < 1) return false;
     if (epi == EPI_GLU) return n % 64 == 0 && k % 256 == 0;   // both tile widths
+    if (epi == EPI_ARGMAX) return n % 64 == 0 && k % 512 == 0;
     if (epi != EPI_DEQUANT && epi != EPI_DEQUANT_RES) return false;
     return k % 512 == 0 && (n % 64 == 0 || pk_split_narrow(m, n));
 }
@@ -1002,6 +1010,12 @@ hipError_t launch_gemm_pk(hipStream_t s, int epi, const GemmArgs& a) {
     const QkvRopeArgs f{};
     if (epi == EPI_GLU) {
         TL_KLAUNCH(gemm_pk_glu_kernel<1>, dim3(a.n / 32, (a.m + 127) / 128), block, pk_glu_lds_bytes(1), s, a);
+        return hipGetLastError();
+    }
+    if (epi == EPI_ARGMAX) {
+        if (!a.key) return hipErrorInvalidValue;
+        TL_KLAUNCH((gemm_pk_split_kernel<2, 2, EPI_ARGMAX>), dim3(a.n / 64, (a.m + 63) / 64), block,
+                   pk_split_lds_bytes(2, 2), s, a, f);
         return hipGetLastError();
     }
     const bool res = epi == EPI_DEQUANT_RES;
@@ -1033,10 +1047,12 @@ hipError_t init_gemm_pk_kernels() {
                          (const void*)gemm_pk_split_kernel<1, 5, EPI_DEQUANT_RES>,
                          (const void*)gemm_pk_split_kernel<2, 2, EPI_DEQUANT>,
                          (const void*)gemm_pk_split_kernel<2, 2, EPI_DEQUANT_RES>, (const void*)gemm_pk_glu_kernel<1>,
-                         (const void*)gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>};
+                         (const void*)gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>,
+                         (const void*)gemm_pk_split_kernel<2, 2, EPI_ARGMAX>};
     const size_t bytes[] = {pk_split_lds_bytes(1, 5), pk_split_lds_bytes(1, 5), pk_split_lds_bytes(2, 2),
-                            pk_split_lds_bytes(2, 2), pk_glu_lds_bytes(1), pk_split_lds_bytes(2, 2)};
-    for (int i = 0; i < 6; i++) {
+                            pk_split_lds_bytes(2, 2), pk_glu_lds_bytes(1), pk_split_lds_bytes(2, 2),
+                            pk_split_lds_bytes(2, 2)};
+    for (int i = 0; i < 7; i++) {
         const hipError_t e = hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes[i]);
         if (e != hipSuccess) return e;
     }

@@ -1799,10 +1799,15 @@ __global__ __launch_bounds__(W * 64) void gemm_rows32_kernel(GemmArgs a) {
     constexpr int NB = EPI == EPI_GLU ? 2 : 1;
     extern __shared__ __align__(16) int rows32_lds[];   // [W waves][NB][16][64]
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), col = lane & 31, hi = lane >> 5;
-    const int n0 = blockIdx.x * 32;
+    // more than one row tile (blockIdx.z) and a packed A: the plain epilogues only
+    constexpr bool MT = EPI == EPI_DEQUANT || EPI == EPI_DEQUANT_RES;
+    const int n0 = blockIdx.x * 32, m0 = MT ? blockIdx.z * 32 : 0;
     const int cps = a.k_split >> 5, c0 = blockIdx.y * cps;
     const int kch = min(cps, (a.k >> 5) - c0);   // chunks of this K slice (>= 1)
-    const int8_t* arow = a.a + (int64_t)min(col, a.m - 1) * a.k + (int64_t)c0 * 32 + hi * 16;
+    // A from its packed copy (1 KiB per fragment load) or row-major (32 rows x 32 bytes)
+    const int8_t* arow = MT && a.ap ? a.ap + ((int64_t)blockIdx.z * (a.k >> 5) + c0) * 1024 + lane * 16
+                              : a.a + (int64_t)min(m0 + col, a.m - 1) * a.k + (int64_t)c0 * 32 + hi * 16;
+    const int64_t astep = MT && a.ap ? 1024 : 32;
     const int8_t* wrow[NB];
     if (PK) {
         const int64_t o = ((int64_t)blockIdx.x * (a.k >> 5) + c0) * 1024 + lane * 16;
@@ -1829,7 +1834,7 @@ __global__ __launch_bounds__(W * 64) void gemm_rows32_kernel(GemmArgs a) {
         if constexpr (EPI == EPI_GLU) esw2 = a.ws2[en];
 #pragma unroll
         for (int ii = 0; ii < NI; ii++) {
-            const int i = wave + W * ii, mc = min(8 * (i >> 2) + 4 * hi + (i & 3), a.m - 1);
+            const int i = wave + W * ii, mc = min(m0 + 8 * (i >> 2) + 4 * hi + (i & 3), a.m - 1);
             esx[ii] = a.as[mc];
             if constexpr (EPI == EPI_DEQUANT_RES) eres[ii] = a.residual[(int64_t)mc * a.n + en];
         }
@@ -1876,7 +1881,7 @@ __global__ __launch_bounds__(W * 64) void gemm_rows32_kernel(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < CH; j++) {
             const int cc = min(wave * per + min(j, per - 1), kch - 1);
-            af[j] = ld16(arow + (int64_t)cc * 32);
+            af[j] = ld16(arow + (int64_t)cc * astep);
 #pragma unroll
             for (int b = 0; b < NB; b++) bf[b][j] = ld_nt16(wrow[b] + (int64_t)cc * wstep);
         }
@@ -1900,7 +1905,7 @@ __global__ __launch_bounds__(W * 64) void gemm_rows32_kernel(GemmArgs a) {
 #pragma unroll
     for (int ii = 0; ii < NI; ii++) {
         const int i = wave + W * ii;
-        const int m = 8 * (i >> 2) + 4 * (l >> 5) + (i & 3), n = n0 + (l & 31);
+        const int m = m0 + 8 * (i >> 2) + 4 * (l >> 5) + (i & 3), n = n0 + (l & 31);
         if (EPI == EPI_ARGMAX) {
             // dequantized logit -> 64-bit key; the 32 columns of row m are the
             // 32 lanes of this half-wavefront, whose best key is this tile's key
@@ -1969,15 +1974,17 @@ static hipError_t launch_rows32_w(hipStream_t s, int epi, const GemmArgs& a, dim
     return hipGetLastError();
 }
 
-// M <= 32, K a multiple of 64 and at most 6144; with packed weights (a.wp,
-// and a.wp2 for the GLU) N must be a multiple of 32.  a.k_split (a multiple
+// M <= 32 (kRows32Max with packed or row-major A for the plain epilogues: one
+// workgroup per 32-row tile, blockIdx.z), K a multiple of 64 and at most 6144;
+// with packed weights (a.wp, and a.wp2 for the GLU) N must be a multiple of 32.  a.k_split (a multiple
 // of 32, 0 = K) slices K over gridDim.y workgroups for EPI_ACC.  waves = 8
 // runs 8-wavefront workgroups (packed weights, K slice at most 2048 bytes),
 // else 16.
 hipError_t launch_gemm_rows32(hipStream_t s, int epi, const GemmArgs& args, int32_t waves) {
     GemmArgs a = args;
-    if (a.m < 1 || a.m > 32 || a.n <= 0 || a.k <= 0 || a.k % 64 || a.k > kRowsWaves * kRowsChunks * 32)
+    if (a.m < 1 || a.m > kRows32Max || a.n <= 0 || a.k <= 0 || a.k % 64 || a.k > kRowsWaves * kRowsChunks * 32)
         return hipErrorInvalidValue;
+    if (epi != EPI_DEQUANT && epi != EPI_DEQUANT_RES && (a.m > 32 || a.ap)) return hipErrorInvalidValue;
     if (a.k_split <= 0 || a.k_split >= a.k || (epi != EPI_ACC && epi != EPI_ACC_F32)) a.k_split = a.k;
     if (a.k_split % 32) return hipErrorInvalidValue;
     if ((epi == EPI_ACC || epi == EPI_ACC_F32) && !a.acc) return hipErrorInvalidValue;
@@ -1990,7 +1997,8 @@ hipError_t launch_gemm_rows32(hipStream_t s, int epi, const GemmArgs& args, int3
                                    (uintptr_t)a.amax % 16 || !a.as_out || a.k_split / 32 > kRowsWaves ||
                  a.k % 4 || (uintptr_t)a.af % 16))
         return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((a.n + 31) / 32), (unsigned)((a.k + a.k_split - 1) / a.k_split));
+    const dim3 grid((unsigned)((a.n + 31) / 32), (unsigned)((a.k + a.k_split - 1) / a.k_split),
+                    (unsigned)((a.m + 31) / 32));
     if (pk && waves == 8 && a.k_split <= 64 * 32 && epi != EPI_ACC_F32) return launch_rows32_w<8>(s, epi, a, grid);
     const dim3 block(1024);
     const size_t lds1 = rows32_lds_bytes(1), lds2 = rows32_lds_bytes(2);

@@ -390,6 +390,18 @@ static int rows32_waves(int epi) {
     return epi == EPI_GLU ? 8 : 16;
 }
 
+// Packed one-matrix GEMMs of few rows: 32 x 32 tiles of 16 wavefronts
+// (launch_gemm_rows32) put more CUs at work than the 64 x 64 tiles of
+// launch_gemm_pk while they run in one round: two workgroups per CU at
+// K <= 2048, one with the 12-chunk variant.  O at 33 to 256 rows 4.2-5.8 us
+// against 5.7-6.2, down at 33 to 128 rows 5.6-6.1 against 9.6 (at 160 rows, two
+// rounds, 10.4 against 9.6).  Gate/up stays with its own kernel (9.9-10.3 us at
+// 33 to 128 rows; 32 x 32 tiles 10.6-17).
+static bool pk_rows32(int epi, int32_t m, int32_t n, int32_t k) {
+    return epi != EPI_GLU && m <= kRows32Max && n % 32 == 0 && k % 64 == 0 && k <= 6144 &&
+           (int64_t)(n / 32) * ((m + 31) / 32) <= (k <= 2048 ? 512 : 256);
+}
+
 int32_t run_gemm(tl_handle* h, int epi, GemmArgs a, int kclass, const FixedScratch* fx = nullptr) {
     const int nb = epi == EPI_GLU ? 2 : 1;
     const bool prof_ok = fx == nullptr;   // profiling events are allocations
@@ -397,7 +409,8 @@ int32_t run_gemm(tl_handle* h, int epi, GemmArgs a, int kclass, const FixedScrat
     if (a.ap) {
         // A was written in the packed operand layout for this GEMM
         Prof p(h, kclass, bytes, prof_ok);
-        TL_LAUNCH(h, launch_gemm_pk(h->stream, epi, a));
+        if (pk_rows32(epi, a.m, a.n, a.k)) TL_LAUNCH(h, launch_gemm_rows32(h->stream, epi, a, rows32_waves(epi)));
+        else TL_LAUNCH(h, launch_gemm_pk(h->stream, epi, a));
         return TL_OK;
     }
     if (a.m >= 64) {
@@ -640,7 +653,7 @@ static int32_t discard_pending_sums(tl_handle* h) {
 // row kernels then write h->a8 in the packed layout those GEMMs read
 static bool prefill_packed(const tl_handle* h, const LayerDev& L, int32_t rows) {
     const int D = h->D, F = h->F, QKV = h->QKV;
-    return rows >= 64 && L.wqkv_p && L.wo_p && L.wg_p && L.wu_p && L.wd_p &&
+    return rows > 32 && L.wqkv_p && L.wo_p && L.wg_p && L.wu_p && L.wd_p &&
            D % 64 == 0 && F % 64 == 0 && D <= 6144 && F <= 6144 && h->plan.n_leaves <= 64 &&
            gemm_pk_supported(EPI_DEQUANT, rows, QKV, D) && gemm_pk_supported(EPI_DEQUANT_RES, rows, D, D) &&
            gemm_pk_supported(EPI_GLU, rows, F, D) && gemm_pk_supported(EPI_DEQUANT_RES, rows, D, F);
@@ -686,7 +699,7 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
     // 32-byte K chunk per wavefront of the 16-wavefront small-M GEMM)
     const bool of = qks && h->o_fuse && L.wo_p && c.n_heads <= 32 && c.n_heads % 4 == 0 &&
                     kslice_len(D, D) / 32 <= 16;
-    const bool pk = !decode && prefill_packed(h, L, rows);   // h->a8 in the packed GEMM operand layout
+    const bool pk = (!decode || rows > 32) && prefill_packed(h, L, rows);   // h->a8 in the packed GEMM operand layout
     // prefill tiles on packed operands: qkv_post's work in the Q|K|V GEMM
     // epilogue, rotated Q in h->qkv ([rows][D]) quantized by the attention tiles
     const bool fq = pk && h->rows_one_seq && h->rows_pos0 + rows <= kTileMaxKeys && D % 64 == 0 &&
@@ -708,10 +721,11 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
         return p;
     };
     const bool l2pf = ks || pk;
-    const int tc = pk ? 64 : 32;
-    const L2Prefetch pf_qkv = pf_plan(L.wqkv_p, nullptr, 1, tc, QKV, D), pf_o = pf_plan(L.wo_p, nullptr, 1, tc, D, D),
-                     pf_glu = pf_plan(L.wg_p, L.wu_p, 2, 32, F, D), pf_down = pf_plan(L.wd_p, nullptr, 1, tc, D, F);
-    const L2Prefetch* pfq = l2pf && (ks || fq) ? &pf_qkv : nullptr;   // prefill: the RoPE-epilogue tiles
+    auto tc = [&](int n, int k) { return pk && !pk_rows32(EPI_DEQUANT, rows, n, k) ? 64 : 32; };
+    const bool q32 = pk && !fq && pk_rows32(EPI_DEQUANT, rows, QKV, D);
+    const L2Prefetch pf_qkv = pf_plan(L.wqkv_p, nullptr, 1, fq ? 64 : 32, QKV, D), pf_o = pf_plan(L.wo_p, nullptr, 1, tc(D, D), D, D),
+                     pf_glu = pf_plan(L.wg_p, L.wu_p, 2, 32, F, D), pf_down = pf_plan(L.wd_p, nullptr, 1, tc(D, F), D, F);
+    const L2Prefetch* pfq = l2pf && (ks || fq || q32) ? &pf_qkv : nullptr;   // prefill: the RoPE-epilogue tiles
     int32_t r;
     if (!ks && (r = discard_pending_sums(h))) return r;
     if ((r = rows_rmsnorm(h, rows, L.g_in, pk, pfq))) return r;
@@ -835,6 +849,7 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
         Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + D * 8.0);
         TL_LAUNCH(h, launch_gemv_fused(h->stream, PRO_RMSNORM, EPI_ARGMAX, g));
     } else {
+        const bool lm_pk = rows > 32 && h->lm_wp && h->plan.n_leaves <= 64 && gemm_pk_supported(EPI_ARGMAX, rows, V, D);
         if (h->racc_res_ws && xrow == h->x) {
             int32_t r = rows_rmsnorm(h, rows, h->g_final);
             if (r) return r;
@@ -842,11 +857,12 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
             int32_t r = discard_pending_sums(h);
             if (r) return r;
             Prof p(h, TL_K_NORM, (double)rows * D * 9.0);
-            TL_LAUNCH(h, launch_rmsnorm_quant(h->stream, xrow, h->g_final, rows, D, c.rms_eps, h->plan, nullptr, h->a8, h->as));
+            TL_LAUNCH(h, launch_rmsnorm_quant(h->stream, xrow, h->g_final, rows, D, c.rms_eps, h->plan, nullptr, h->a8, h->as, lm_pk));
         }
         GemmArgs a{};
+        if (lm_pk) a.ap = h->a8;
         a.a = h->a8; a.w = h->lm_w; a.as = h->as; a.ws = h->lm_s; a.y = h->logits; a.m = rows; a.n = V; a.k = D;
-        if (rows <= 32 && h->lm_wp && D % 64 == 0 && D <= 2048) {
+        if (lm_pk || (rows <= 32 && h->lm_wp && D % 64 == 0 && D <= 2048)) {
             // packed-weight MFMA GEMM with the argmax in its epilogue (one key
             // per 32-column tile and row), then the tiles' keys folded per row
             const int tiles = V / 32;
@@ -856,7 +872,8 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
             a.key = (unsigned long long*)h->partials;
             a.y = nullptr;
             Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + (double)rows * D);
-            TL_LAUNCH(h, launch_gemm_rows32(h->stream, EPI_ARGMAX, a, rows32_waves(EPI_ARGMAX)));
+            if (lm_pk) TL_LAUNCH(h, launch_gemm_pk(h->stream, EPI_ARGMAX, a));
+            else TL_LAUNCH(h, launch_gemm_rows32(h->stream, EPI_ARGMAX, a, rows32_waves(EPI_ARGMAX)));
             TL_LAUNCH(h, launch_argmax_tiles(h->stream, a.key, tiles, rows, keys));
         } else {
             // MFMA GEMM writes logits, a row argmax folds them into keys

@@ -1,0 +1,94 @@
+"""GPU parity between the 32-row tile and the large tiles: batches and prompts of 33 to 300 rows, and the context
+bounds of the batched attention."""
+from __future__ import annotations
+
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+from gpu_util import assert_bits_equal, dev, host
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+
+
+def _fill(eng, cfg, seq, n, rng, kc, vc):
+    for layer in range(cfg["n_layers"]):
+        for g in range(cfg["n_kv_heads"]):
+            kc[layer, g, :n] = np.clip(np.rint(rng.standard_normal((n, 64)) * 25), -127, 127)
+            vc[layer, g, :n] = np.clip(np.rint(rng.standard_normal((n, 64)) * 25), -127, 127)
+            eng.kv_write(seq, layer, g, 0, kc[layer, g, :n], vc[layer, g, :n])
+
+
+@pytest.mark.parametrize("B,top", [(33, 505), (64, 1017), (90, 300), (128, 70), (129, 90), (3, 510)])
+def test_decode_batch_rows_and_context_bounds(B, top):
+    """Batches past 32 rows (32 x 32 tiles of several row tiles, their last
+    one partial; LM-head argmax keys of 64-column tiles) with ragged contexts up
+    to `top` cached rows, so that a second call of the same batch crosses the
+    bound of 512 or 1024 keys (another captured step, another wavefront count
+    of the grouped attention): ids and appended K/V rows equal the oracle's."""
+    from lpta.engine import Engine
+    cfg = dict(oracle.TINYLLAMA_CFG, n_layers=1, vocab=512)
+    m = oracle.synthetic_model(cfg, seed=70 + B)
+    eng = Engine(m.cfg, max_seqs=B).load_model(m)
+    rng = np.random.default_rng(B)
+    start = rng.integers(max(1, top - 60), top + 1, B).astype(np.int32)
+    start[0], start[-1] = top, 1
+    toks = rng.integers(0, cfg["vocab"], B).astype(np.int32)
+    caches = []
+    for b in range(B):
+        kc, vc = m.new_cache()
+        _fill(eng, cfg, b, int(start[b]), rng, kc, vc)
+        caches.append((kc, vc))
+    oracle.lib().or_set_threads(max(1, min(16, len(os.sched_getaffinity(0)))))
+    orc = oracle.Oracle(m)
+    pos, tok = start.copy(), toks
+    for steps in (3, 5):   # one eager step and replays; the second call ends past the bound for top = 505, 1017, 510
+        got = eng.decode_batch(tok, pos, steps)
+        for s in range(steps):
+            x = np.stack([orc.embed(int(t)) for t in tok]).astype(F32)
+            orc.decode_rows(0, pos, x, caches)
+            tok, _ = orc.lm_head_rows(x)
+            tok = np.asarray(tok, np.int32)
+            assert_bits_equal(np.asarray(got[:, s], np.int32), tok, f"ids of step {s}")
+            pos = pos + 1
+    for b in (0, 1, 31, 32, B // 2, B - 1):
+        if b >= B:
+            continue
+        kc, vc = caches[b]
+        n = int(pos[b])
+        for g in range(cfg["n_kv_heads"]):
+            k, v = eng.kv_read(b, 0, g, 0, n)
+            assert_bits_equal(k, kc[0, g, :n], f"K seq {b} head {g}")
+            assert_bits_equal(v, vc[0, g, :n], f"V seq {b} head {g}")
+    eng.close()
+
+
+@pytest.fixture(scope="module")
+def layer_eng():
+    from lpta.engine import Engine
+    e = Engine(dict(oracle.TINYLLAMA_CFG, n_layers=1, vocab=64), max_seqs=2)
+    e.load_random(11)
+    yield e
+    e.close()
+
+
+@pytest.mark.parametrize("rows", [32, 33, 63, 64, 65, 128, 129, 256, 257, 300])
+def test_layer_rows_equal_single_rows(layer_eng, rows):
+    """Both sides of every row count at which a projection changes kernel: the
+    layer over all rows equals the single-row kernels run row after row on
+    another sequence, output and cache."""
+    d = oracle.TINYLLAMA_CFG["hidden"]
+    x = np.random.default_rng(rows).standard_normal((rows, d)).astype(F32)
+    xs = dev(x)
+    layer_eng.rt.call("tl_layer_rows", 0, 0, 0, rows, xs)
+    got = host(xs)
+    one = dev(x)
+    for r in range(rows):
+        layer_eng.decode_layer(one[r], 0, r, seq=1)
+    assert_bits_equal(got, host(one), f"{rows} rows")
+    for g in range(4):
+        for a, b in zip(layer_eng.kv_read(0, 0, g, 0, rows), layer_eng.kv_read(1, 0, g, 0, rows)):
+            assert_bits_equal(a, b, f"cache head {g}")
