@@ -644,34 +644,35 @@ __global__ __launch_bounds__(256) void attention_row_kernel(AttnDecodeArgs p) {
     }
 }
 
-// Batched decode attention (many rows, long contexts): one workgroup of 16
+// Batched decode attention (many rows): one workgroup of NWV = 4, 8 or 16
 // wavefronts per (row, group of HPW = 4 query heads sharing a KV head).  The
 // Q.K scores and the P.V sums run on v_mfma_i32_16x16x64_i8 with the four
 // heads as rows 0, 4, 8 and 12 of the 16-row A operand (the other rows zero),
 // so accumulator register 0 of lane l holds head l / 16 at column l % 16: a
 // wavefront keeps every (head, key) value it computes in all 64 lanes, one
-// 16-lane row per head.  Wavefront w owns key blocks b = w + 16 i (64 keys,
+// 16-lane row per head.  Wavefront w owns key blocks b = w + NWV i (64 keys,
 // i < 2): per block four MFMAs of 16 keys for the scores (lane l: keys
 // 16 j + l % 16, j < 4, of head l / 16) and, per 16 output dimensions, one
 // MFMA over the block's 64 keys for P.V.  Every wavefront issues all of its
-// key and value loads first (T <= 2048), so each phase costs about one
+// key and value loads first (T <= 128 NWV), so each phase costs about one
 // memory latency.  Same arithmetic as attention_row_kernel: the integer dot
 // products are exact in any order, and the block sums keep the block-64
 // butterfly order (levels 32 and 16 inside a lane's registers, 8, 4, 2, 1
 // across its row).
-constexpr int kGW = 16;                         // wavefronts
+constexpr int kGW = 16;                         // most wavefronts
 constexpr int kGKB = 2;                         // key blocks of 64 per wavefront
 constexpr int kGroupMaxKeys = kGW * kGKB * 64;  // 2048
+constexpr int group_max_keys(int w) { return w * kGKB * 64; }
 
-template <int HPW>
-__global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArgs p) {
+template <int HPW, int NWV>
+__global__ __launch_bounds__(NWV * 64) void attention_group_kernel(AttnDecodeArgs p) {
     static_assert(HPW == 4, "one head per 16-lane row of the MFMA accumulators");
     extern __shared__ __align__(16) float gdyn[];
     __shared__ __align__(16) int8_t qs[HPW][64];
     __shared__ __align__(16) int8_t kn[64];
     __shared__ __align__(16) int8_t vn[64];
-    __shared__ float red[kGW];
-    __shared__ float wmax[kGW][HPW];
+    __shared__ float red[NWV];
+    __shared__ float wmax[NWV][HPW];
     __shared__ float mh[HPW], toth[HPW];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
@@ -701,7 +702,7 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     const int8_t* vp = p.kv.v + pl;
     int8_t* p8 = (int8_t*)gdyn;                           // [HPW][tpad]
     float* bsum = (float*)(p8 + HPW * tpad);              // [HPW][nblk]
-    int* accs = (int*)(bsum + HPW * nblk);                // [kGW][HPW][64]
+    int* accs = (int*)(bsum + HPW * nblk);                // [NWV][HPW][64]
     const bool sums = p.qacc != nullptr;   // uniform
     const double qsx = sums ? p.qas[row] : 0.0;
     // one load path for both forms, so that no load waits on another: the
@@ -729,12 +730,12 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     //    one before the probabilities, where their issue delays less:
     //    measured per workgroup at 2048 keys, 13.4 us with every load at the
     //    start, 11.9 with all value loads before the scores, 11.4 split
-    constexpr int kQPer = 4;   // Q elements per thread: D <= 4 x 1024
+    constexpr int kQPer = 64 / NWV;   // Q elements per thread: D <= 4096
     int32_t qw[kQPer + 3];
     float qm[kQPer + 3];
 #pragma unroll
     for (int j = 0; j < kQPer; j++) {
-        const int i = min(tid + kGW * 64 * j, D - 1);
+        const int i = min(tid + NWV * 64 * j, D - 1);
         qw[j] = srcw[i];
         qm[j] = srcm[i];
     }
@@ -752,12 +753,12 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     v4i kreg[kGKB][4], vreg[kGKB][4];
 #pragma unroll
     for (int i = 0; i < kGKB; i++) {
-        const int b = min(wave + kGW * i, nblk - 1);
+        const int b = min(wave + NWV * i, nblk - 1);
 #pragma unroll
         for (int j = 0; j < 4; j++) kreg[i][j] = ld16(kp + (int64_t)b * 4096 + hl * 1024 + (16 * j + cl) * 16);
     }
     auto v_load = [&](int i) {
-        const int b = min(wave + kGW * i, nblk - 1);
+        const int b = min(wave + NWV * i, nblk - 1);
 #pragma unroll
         for (int j = 0; j < 4; j++) vreg[i][j] = ld16(vp + (int64_t)(4 * b + hl) * 1024 + (16 * j + cl) * 16);
     };
@@ -775,7 +776,7 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
 #pragma unroll
     for (int j = 0; j < kQPer; j++) {
         const float o = lane_xor<32>(qv[j]);
-        if (tid + kGW * 64 * j < D) mx = fmaxf(mx, fabsf((qv[j] * cs) + ((d < 32 ? -o : o) * sn)));
+        if (tid + NWV * 64 * j < D) mx = fmaxf(mx, fabsf((qv[j] * cs) + ((d < 32 ? -o : o) * sn)));
     }
     mx = wave_max_f32(mx);
     if (lane == 0) red[wave] = mx;
@@ -783,13 +784,14 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     __syncthreads();
     mx = red[0];
 #pragma unroll
-    for (int w = 1; w < kGW; w++) mx = fmaxf(mx, red[w]);
+    for (int w = 1; w < NWV; w++) mx = fmaxf(mx, red[w]);
     const double s_q = quant_scale(mx);
     if (wave < HPW) {
         const float qo = lane_xor<32>(qh);
         const float qr = (qh * cs) + ((d < 32 ? -qo : qo) * sn);
         qs[wave][d] = sat_i8(__builtin_rintf(__fdiv_rn(qr, (float)s_q)));
-    } else if (wave == HPW) {
+    }
+    if (wave == (NWV > HPW ? HPW : 0)) {   // a wavefront of its own where there is one
         const float ko = lane_xor<32>(kx);
         const float kr = (kx * cs) + ((d < 32 ? -ko : ko) * sn);
         const int8_t k8 = sat_i8(__builtin_rintf(__fdiv_rn(kr, sk)));
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     float lmax = -INFINITY;
 #pragma unroll
     for (int i = 0; i < kGKB; i++) {
-        const int b = wave + kGW * i;
+        const int b = wave + NWV * i;
         if (b < nblk) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -838,7 +840,7 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     __syncthreads();
     if (tid < HPW) {
         float m = wmax[0][tid];
-        for (int w = 1; w < kGW; w++) m = fmaxf(m, wmax[w][tid]);
+        for (int w = 1; w < NWV; w++) m = fmaxf(m, wmax[w][tid]);
         mh[tid] = m;
     }
     __syncthreads();
@@ -849,7 +851,7 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     const float mhh = mh[hl];
 #pragma unroll
     for (int i = 0; i < kGKB; i++) {
-        const int b = wave + kGW * i;
+        const int b = wave + NWV * i;
         if (b < nblk) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -888,7 +890,7 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     auto probs = [&](auto fst) {
 #pragma unroll
         for (int i = 0; i < kGKB; i++) {
-            const int b = wave + kGW * i;
+            const int b = wave + NWV * i;
             if (b < nblk) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -914,7 +916,7 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     const int gpos = pos >> 4, bq = (pos & 15) >> 2, bsh = (pos & 3) * 8;
 #pragma unroll
     for (int i = 0; i < kGKB; i++) {
-        const int b = wave + kGW * i;
+        const int b = wave + NWV * i;
         if (b < nblk) {
             const v4i prow = *(const v4i*)(p8 + (cl >> 2) * tpad + b * 64 + 16 * hl);
             const v4i pa = (cl & 3) == 0 ? prow : vzero;
@@ -938,7 +940,7 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     if (tid < HPW * 64) {   // wavefront h: head h0 + h
         const int h = tid >> 6, dd = tid & 63;
         int O = 0;
-        for (int w = 0; w < kGW; w++) O += accs[(w * HPW + h) * 64 + dd];
+        for (int w = 0; w < NWV; w++) O += accs[(w * HPW + h) * 64 + dd];
         const float v = (float)O * deq_mult(1.0 / 127.0, sv);
         p.out[(int64_t)row * D + (int64_t)(h0 + h) * kHeadDim + dd] = v;
         if (p.out_max) {   // the head's part of the maximum the O projection quantizes the row at
@@ -948,8 +950,8 @@ __global__ __launch_bounds__(kGW * 64) void attention_group_kernel(AttnDecodeArg
     }
 }
 
-static size_t group_lds_bytes(int hpw, int tpad) {
-    return (size_t)hpw * tpad + (size_t)hpw * (tpad / 64) * 4 + (size_t)kGW * hpw * 64 * 4 + 16;
+static size_t group_lds_bytes(int hpw, int tpad, int w) {
+    return (size_t)hpw * tpad + (size_t)hpw * (tpad / 64) * 4 + (size_t)w * hpw * 64 * 4 + 16;
 }
 
 // embedding of each row's current token and the row's position (= its
@@ -1068,8 +1070,16 @@ hipError_t launch_attention_decode(hipStream_t s, const float* qkv, int32_t rows
         // many rows: the grouped kernel, 4 query heads per workgroup (with 8
         // per workgroup, one per KV head, it measured slower: half the
         // workgroups, longer phases)
-        TL_KLAUNCH((attention_group_kernel<4>), dim3(n_heads / 4, rows), dim3(kGW * 64), group_lds_bytes(4, tpad), s,
-                   p);
+        // as few wavefronts as hold the context at two key blocks each: more
+        // workgroups fit on a CU and fewer wavefronts idle at its barriers
+        // (90 rows x 260 keys 10.2 us against 19.8 with 16 wavefronts, 128 x 200
+        // 10.9 against 25.2; 64 x 900 11.8 with 8 against 17.5)
+        const dim3 grid(n_heads / 4, rows);
+        if (max_t <= group_max_keys(4))
+            TL_KLAUNCH((attention_group_kernel<4, 4>), grid, dim3(256), group_lds_bytes(4, tpad, 4), s, p);
+        else if (max_t <= group_max_keys(8))
+            TL_KLAUNCH((attention_group_kernel<4, 8>), grid, dim3(512), group_lds_bytes(4, tpad, 8), s, p);
+        else TL_KLAUNCH((attention_group_kernel<4, kGW>), grid, dim3(kGW * 64), group_lds_bytes(4, tpad, kGW), s, p);
     } else if (n_heads % 4 == 0 && D <= kRowQPerThread * kNT) {
         const size_t lds = (size_t)tpad * 5 + (tpad / 64) * 4 + 16;
         TL_KLAUNCH((attention_row_kernel<2>), dim3(n_heads, rows), dim3(256), lds, s, p);
@@ -1093,8 +1103,8 @@ hipError_t init_decode_kernels() {
     hipError_t e = hipFuncSetAttribute((const void*)attention_row_kernel<2>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024);
     if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)attention_group_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)group_lds_bytes(4, kGroupMaxKeys));
+    e = hipFuncSetAttribute((const void*)attention_group_kernel<4, kGW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)group_lds_bytes(4, kGroupMaxKeys, kGW));
     if (e != hipSuccess) return e;
     return hipFuncSetAttribute((const void*)attention_decode_kernel<1, 2, 8, 4>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);

@@ -199,7 +199,7 @@ struct tl_handle {
     bool rows_one_seq = false;            // the uploaded rows are one sequence at rows_pos0 + r
     int32_t rows_seq = 0, rows_pos0 = 0;
     std::vector<hipGraphExec_t> graphs;   // captured batch-1 decode step per sequence
-    std::vector<hipGraphExec_t> batch_graphs;   // captured batched decode step, by batch size
+    std::vector<hipGraphExec_t> batch_graphs;   // captured batched decode step, by batch size and context bucket
 
     bool profiling = false;
     // decode timeline: while ts_on, the launches of a step take consecutive
@@ -1012,13 +1012,22 @@ int32_t batch_step(tl_handle* h, int32_t n_seqs, int32_t max_t) {
     return lm_head_rows(h, h->x, n_seqs, 0, 1);
 }
 
-// replay of the captured batched step (captured on first use for this batch
-// size, with the attention sized for the whole context)
-int32_t batch_graph_launch(tl_handle* h, int32_t n_seqs) {
-    if ((int)h->batch_graphs.size() <= h->max_seqs) h->batch_graphs.resize(h->max_seqs + 1, nullptr);
-    if (!h->batch_graphs[n_seqs]) {
+// context bounds the batched step is captured for: the attention launch
+// depends on its bound (wavefronts per workgroup, grouped kernel or not)
+constexpr int kCtxBuckets = 4;
+constexpr int32_t kCtxBound[kCtxBuckets - 1] = {512, 1024, 2048};
+
+// replay of the captured batched step for positions below max_t (captured on
+// first use for this batch size and context bucket)
+int32_t batch_graph_launch(tl_handle* h, int32_t n_seqs, int32_t max_t) {
+    int bucket = 0;
+    while (bucket < kCtxBuckets - 1 && max_t > kCtxBound[bucket]) bucket++;
+    const int32_t bound = bucket < kCtxBuckets - 1 ? std::min(kCtxBound[bucket], h->cfg.max_pos) : h->cfg.max_pos;
+    if (h->batch_graphs.empty()) h->batch_graphs.resize((size_t)(h->max_seqs + 1) * kCtxBuckets, nullptr);
+    hipGraphExec_t& exec = h->batch_graphs[(size_t)n_seqs * kCtxBuckets + bucket];
+    if (!exec) {
         TL_HIP(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        int32_t r = batch_step(h, n_seqs, h->cfg.max_pos);
+        int32_t r = batch_step(h, n_seqs, bound);
         hipGraph_t cap = nullptr;
         hipError_t e = hipStreamEndCapture(h->stream, &cap);
         if (r) {
@@ -1030,9 +1039,9 @@ int32_t batch_graph_launch(tl_handle* h, int32_t n_seqs) {
         e = hipGraphInstantiate(&ex, cap, nullptr, nullptr, 0);
         (void)hipGraphDestroy(cap);
         TL_HIP(h, e);
-        h->batch_graphs[n_seqs] = ex;
+        exec = ex;
     }
-    TL_HIP(h, hipGraphLaunch(h->batch_graphs[n_seqs], h->stream));
+    TL_HIP(h, hipGraphLaunch(exec, h->stream));
     return TL_OK;
 }
 
@@ -1899,7 +1908,7 @@ int32_t tl_decode_batch(tl_handle* h, int32_t n_seqs, const int32_t* tokens, con
     // keys need), the rest replay the captured step
     for (int step = 0; step < n_steps; step++) {
         if (step > 0 && !h->profiling) {
-            if ((r = batch_graph_launch(h, n_seqs))) return r;
+            if ((r = batch_graph_launch(h, n_seqs, max_t))) return r;
         } else if ((r = batch_step(h, n_seqs, max_t))) {
             return r;
         }
