@@ -632,8 +632,8 @@ TL_DEV void qkv_rope_operands(const GemmArgs& a, const QkvRopeArgs& f, int mt0, 
     for (int ee = 0; ee < NE; ee++) {
         const int e = o.e0 + ee, m = min(o.rb + 8 * (e >> 2) + (e & 3), a.m - 1);
         o.sx[ee] = a.as[m];
-        o.pos[ee] = f.rm.pos[m];
-        o.seq[ee] = f.rm.seq[m];
+        o.pos[ee] = f.rm.pos_of(m);
+        o.seq[ee] = f.rm.seq_of(m);
     }
 }
 

@@ -44,11 +44,16 @@ struct KvGeom {
     }
 };
 
-// Per-row description used by the row-parallel kernels (prefill rows of one
-// sequence, or one row per sequence in batched decode).
+// Per-row description used by the row-parallel kernels: rows of one sequence at
+// consecutive positions that the host knows (seq and pos null; no memory read
+// before the kernel can form its cache addresses), or arrays (decode steps, whose
+// positions advance on the device; one row per sequence in batched decode).
 struct RowMap {
-    const int32_t* seq;  // [rows] sequence (KV plane) of each row
-    const int32_t* pos;  // [rows] position of each row
+    const int32_t* seq;  // [rows] sequence (KV plane) of each row, or null: seq0
+    const int32_t* pos;  // [rows] position of each row, or null: pos0 + row
+    int32_t seq0, pos0;
+    __host__ __device__ int32_t seq_of(int32_t row) const { return seq ? seq[row] : seq0; }
+    __host__ __device__ int32_t pos_of(int32_t row) const { return pos ? pos[row] : pos0 + row; }
 };
 
 enum GemvEpi : int {

@@ -196,8 +196,9 @@ struct tl_handle {
                                           // at the row maxima the attention kernel leaves; its sums folded by the
                                           // post-attention RMSNorm (TL_BATCH_O_FUSE=0 turns it off)
     bool qmax_clean = true;               // false from a fused Q|K|V GEMM until qmax is cleared
-    bool rows_one_seq = false;            // the uploaded rows are one sequence at rows_pos0 + r
+    bool rows_one_seq = false;            // the rows are one sequence at rows_pos0 + r
     int32_t rows_seq = 0, rows_pos0 = 0;
+    bool rows_on_host = false;            // ... and its kernels take them as arguments (row_seq / row_pos unused)
     std::vector<hipGraphExec_t> graphs;   // captured batch-1 decode step per sequence
     std::vector<hipGraphExec_t> batch_graphs;   // captured batched decode step, by batch size and context bucket
 
@@ -506,9 +507,12 @@ int32_t linear(tl_handle* h, int epi, int rows, const int8_t* x8, const double* 
     return run_gemm(h, epi, a, kclass);
 }
 
-RowMap rowmap(tl_handle* h) { return RowMap{h->row_seq, h->row_pos}; }
+RowMap rowmap(const tl_handle* h) {
+    if (h->rows_on_host) return RowMap{nullptr, nullptr, h->rows_seq, h->rows_pos0};
+    return RowMap{h->row_seq, h->row_pos, 0, 0};
+}
 
-// causal attention of the uploaded rows: MFMA tiles when the rows are one
+// causal attention of the rows set by set_rows: MFMA tiles when the rows are one
 // sequence (prefill), else one workgroup per (row, KV head)
 hipError_t rows_attention(tl_handle* h, const int8_t* q8, const double* q_scale, int32_t rows, int32_t layer,
                           float* out, int32_t max_t) {
@@ -891,20 +895,24 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
     return TL_OK;
 }
 
-// rows 0 .. rows - 1 of the workspaces: their sequences and positions
-RowsInit rows_init(tl_handle* h, int32_t rows, int32_t seq_first, bool seq_per_row, int32_t pos0) {
-    h->rows_one_seq = !seq_per_row;
-    h->rows_seq = seq_first;
+// rows 0 .. rows - 1 of the workspaces are positions pos0 .. of one sequence
+void set_rows(tl_handle* h, int32_t seq, int32_t pos0) {
+    h->rows_one_seq = h->rows_on_host = true;
+    h->rows_seq = seq;
+    h->rows_pos0 = pos0;
+}
+
+// ... or, with their sequences and positions in device memory (decode steps):
+// one row of sequence seq at pos0, or (per_row) row r of sequence seq + r
+RowsInit rows_init(tl_handle* h, int32_t rows, int32_t seq, bool per_row, int32_t pos0) {
+    h->rows_one_seq = !per_row;
+    h->rows_on_host = false;
+    h->rows_seq = seq;
     h->rows_pos0 = pos0;
     RowsInit a{};
     a.row_seq = h->row_seq; a.row_pos = h->row_pos;
-    a.rows = rows; a.seq = seq_first; a.pos0 = pos0; a.per_row = seq_per_row;
+    a.rows = rows; a.seq = seq; a.pos0 = pos0; a.per_row = per_row;
     return a;
-}
-
-int32_t set_rows(tl_handle* h, int32_t rows, int32_t seq_first, bool seq_per_row, int32_t pos0) {
-    TL_LAUNCH(h, launch_rows_init(h->stream, rows_init(h, rows, seq_first, seq_per_row, pos0)));
-    return TL_OK;
 }
 
 // row 0 of the workspaces for decode steps of sequence seq at position pos,
@@ -1546,8 +1554,7 @@ int32_t tl_qkv_append(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, in
     TL_REQ(h, rows >= 1 && rows <= h->max_rows && pos0 >= 0 && (int64_t)pos0 + rows <= c.max_pos,
            "position range out of bounds");
     TL_REQ(h, qkv && q8 && q_scale, "null pointer");
-    int32_t r = set_rows(h, rows, seq, false, pos0);
-    if (r) return r;
+    set_rows(h, seq, pos0);
     TL_LAUNCH(h, launch_qkv_post(h->stream, qkv, rows, c.n_heads, c.n_kv_heads, rowmap(h), h->rope_cos, h->rope_sin,
                                  h->kv, layer, h->kv_sk, h->kv_sv, q8, q_scale, q_rot));
     return finish(h);
@@ -1561,8 +1568,7 @@ int32_t tl_attention(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, int
     TL_REQ(h, rows >= 1 && rows <= h->max_rows && pos0 >= 0 && (int64_t)pos0 + rows <= c.max_pos,
            "position range out of bounds");
     TL_REQ(h, q8 && q_scale && out, "null pointer");
-    int32_t r = set_rows(h, rows, seq, false, pos0);
-    if (r) return r;
+    set_rows(h, seq, pos0);
     {
         Prof p(h, TL_K_ATTN, 0.0);
         TL_LAUNCH(h, rows_attention(h, q8, q_scale, rows, layer, out, pos0 + rows));
@@ -1636,8 +1642,8 @@ int32_t tl_decode_layer(tl_handle* h, int32_t seq, int32_t layer, int32_t pos, f
     TL_REQ(h, pos >= 0 && pos < c.max_pos, "position out of range");
     TL_REQ(h, x, "null pointer");
     if (!h->layers[layer].wqkv) return fail(h, TL_ERR_BAD_DESCRIPTOR, "layer not loaded");
-    int32_t r = set_rows(h, 1, seq, false, pos);
-    if (r) return r;
+    int32_t r;
+    set_rows(h, seq, pos);
     const CallerRows cx(h, x, 1);
     TL_HIP(h, cx.in());
     if ((r = layer_rows(h, layer, 1, pos + 1, true))) return r;
@@ -1666,7 +1672,8 @@ int32_t prefill_layers(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t
     h->host_ngen[seq] = 0;   // the sequence is rewritten: no decode until prefill_finish
     h->host_cursor[seq] = 0;
     TL_HIP(h, hipMemcpyAsync(h->tokens, tokens, sizeof(int32_t) * n, hipMemcpyHostToDevice, h->stream));
-    RowsInit init = rows_init(h, n, seq, false, 0);
+    set_rows(h, seq, 0);
+    RowsInit init{};   // the sequence's state only
     init.n_gen = h->n_gen + seq; init.cursor = h->cursor + seq; init.cursor_v = n;
     init.key = h->keys + seq;
     init.eos = h->eos_id + seq; init.eos_v = -1;
@@ -1743,8 +1750,8 @@ int32_t tl_layer_rows(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, in
     TL_REQ(h, pos0 >= 0 && (int64_t)pos0 + rows <= c.max_pos, "Sequence length exceeds max_position_embeddings");
     TL_REQ(h, x, "null pointer");
     if (!h->layers[layer].wqkv) return fail(h, TL_ERR_BAD_DESCRIPTOR, "layer not loaded");
-    int32_t r = set_rows(h, rows, seq, false, pos0);
-    if (r) return r;
+    int32_t r;
+    set_rows(h, seq, pos0);
     const CallerRows cx(h, x, rows);
     TL_HIP(h, cx.in());
     if ((r = layer_rows(h, layer, rows, pos0 + rows, rows == 1))) return r;
@@ -1898,7 +1905,7 @@ int32_t tl_decode_batch(tl_handle* h, int32_t n_seqs, const int32_t* tokens, con
     }
     int32_t r = check_model_loaded(h);
     if (r) return r;
-    if ((r = set_rows(h, n_seqs, 0, true, 0))) return r;
+    TL_LAUNCH(h, launch_rows_init(h->stream, rows_init(h, n_seqs, 0, true, 0)));
     std::vector<int32_t> zeros(n_seqs, 0);
     TL_HIP(h, hipMemcpyAsync(h->token_cur, tokens, sizeof(int32_t) * n_seqs, hipMemcpyHostToDevice, h->stream));
     TL_HIP(h, hipMemcpyAsync(h->cursor, start_pos, sizeof(int32_t) * n_seqs, hipMemcpyHostToDevice, h->stream));
