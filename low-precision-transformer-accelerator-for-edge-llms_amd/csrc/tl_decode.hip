@@ -424,11 +424,12 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnDecodeArg
 // INT8 Q and of this row's INT8 K (lane d <-> dimension d; RoPE's partner
 // dimension d ^ 32 is lane d ^ 32 of the same wavefront).
 // ---------------------------------------------------------------------------
-constexpr int kRowQPerThread = 16;   // Q width <= 16 x 256
+constexpr int kRowMaxD = 4096;   // widest Q row
 
-template <int KPF>
-__global__ __launch_bounds__(256) void attention_row_kernel(AttnDecodeArgs p) {
-    constexpr int NW = 4, KB = 4;
+template <int KPF, int NW>
+__global__ __launch_bounds__(NW * 64) void attention_row_kernel(AttnDecodeArgs p) {
+    constexpr int KB = 4, NT = NW * 64, kQPer = kRowMaxD / NT;
+    constexpr bool VLATE = NW == 16;   // 128 registers per lane: the value rows are requested after the scores
     extern __shared__ __align__(16) float dyn[];
     __shared__ __align__(16) int8_t qs[NW][64];
     __shared__ __align__(16) int8_t kn[NW][64];
@@ -460,14 +461,13 @@ __global__ __launch_bounds__(256) void attention_row_kernel(AttnDecodeArgs p) {
     const int d = lane;
 
     // 1) RoPE factors, every Q element (the row's scale is the max over all
-    //    heads; element tid + 256 j has dimension d), this head's Q, this
+    //    heads; element tid + NT j has dimension d), this head's Q, this
     //    row's K and V (clamped, in-bounds indices) ...
     const float cs = p.cosb[(int64_t)pos * kHeadDim + d];
     const float sn = p.sinb[(int64_t)pos * kHeadDim + d];
-    const int nq = D / kNT;   // D is a multiple of 256 (64 x heads, heads % 4 == 0 checked at launch)
-    float qv[kRowQPerThread];
+    float qv[kQPer];
 #pragma unroll
-    for (int j = 0; j < kRowQPerThread; j++) qv[j] = src[min(tid + kNT * j, D - 1)];
+    for (int j = 0; j < kQPer; j++) qv[j] = src[min(tid + NT * j, D - 1)];
     const float qh = src[h0 * kHeadDim + d];
     const float kx = src[D + g * kHeadDim + d];
     const float vx = src[D + KVD + g * kHeadDim + d];
@@ -481,18 +481,19 @@ __global__ __launch_bounds__(256) void attention_row_kernel(AttnDecodeArgs p) {
         const int b = min(wave + NW * i, nblk - 1);
 #pragma unroll
         for (int q = 0; q < 4; q++) kreg[i][q] = ld16(kp + (int64_t)b * 4096 + q * 1024 + lane * 16);
+        if (!VLATE)
 #pragma unroll
-        for (int q = 0; q < 4; q++) vreg[i][q] = ld16(vp + (int64_t)(4 * b + q) * 1024 + lane * 16);
+            for (int q = 0; q < 4; q++) vreg[i][q] = ld16(vp + (int64_t)(4 * b + q) * 1024 + lane * 16);
     }
     __builtin_amdgcn_sched_barrier(0);
 
     // 2) RoPE of every Q element -> row maximum
     float mx = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kRowQPerThread; j++) {
+    for (int j = 0; j < kQPer; j++) {
         const float o = lane_xor<32>(qv[j]);
         const float rot = d < 32 ? -o : o;
-        if (j < nq) mx = fmaxf(mx, fabsf((qv[j] * cs) + (rot * sn)));
+        if (tid + NT * j < D) mx = fmaxf(mx, fabsf((qv[j] * cs) + (rot * sn)));
     }
     mx = wave_max_f32(mx);
     if (lane == 0) red[wave] = mx;
@@ -508,7 +509,9 @@ __global__ __launch_bounds__(256) void attention_row_kernel(AttnDecodeArgs p) {
         p.kv.v[pl + KvGeom::v_off(pos, d)] = v8;
     }
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    mx = red[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) mx = fmaxf(mx, red[w]);
     const double s_q = quant_scale(mx);
     qs[wave][d] = sat_i8(__builtin_rintf(__fdiv_rn(qr, (float)s_q)));
     const float scl = (float)((s_q * (double)sk) * p.attn_scale);
@@ -557,10 +560,20 @@ __global__ __launch_bounds__(256) void attention_row_kernel(AttnDecodeArgs p) {
             if (b0 + NW * i < nblk)
                 score_block(b0 + NW * i, kk[i][0], kk[i][1], kk[i][2], kk[i][3], s_buf[(b0 + NW * i) * 64 + lane]);
     }
+    if (VLATE) {   // the key registers are free now
+#pragma unroll
+        for (int i = 0; i < KPF; i++) {
+            const int b = min(wave + NW * i, nblk - 1);
+#pragma unroll
+            for (int q = 0; q < 4; q++) vreg[i][q] = ld16(vp + (int64_t)(4 * b + q) * 1024 + lane * 16);
+        }
+    }
     lmax = wave_max_f32(lmax);
     if (lane == 0) wmax[wave] = lmax;
     __syncthreads();
-    const float m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    float m = wmax[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) m = fmaxf(m, wmax[w]);
 
     // 4) exponentials and block-64 butterfly sums of this wavefront's keys
     auto exp_block = [&](int b, float& x) {
@@ -639,7 +652,9 @@ __global__ __launch_bounds__(256) void attention_row_kernel(AttnDecodeArgs p) {
     accs[wave][lane] = o;
     __syncthreads();
     if (tid < 64) {
-        const int O = accs[0][tid] + accs[1][tid] + accs[2][tid] + accs[3][tid];
+        int O = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) O += accs[w][tid];
         p.out[(int64_t)row * D + (int64_t)h0 * kHeadDim + tid] = (float)O * deq_mult(1.0 / 127.0, sv);
     }
 }
@@ -1040,6 +1055,12 @@ hipError_t launch_gemv_fused(hipStream_t s, int pro, int epi, const GemvArgs& a)
     return hipErrorInvalidValue;
 }
 
+// two 64-key blocks per wavefront in registers: past 512 keys more wavefronts
+// beat a loop over further blocks (701 keys 5.9 us against 7.5 with 4
+// wavefronts, 1024 keys 6.5 against 8.1, 2048 keys 8.0 against 10.7); at 512 and
+// fewer, 4 wavefronts hold every key and the barriers are cheaper
+int32_t attention_row_waves(int32_t max_t) { return max_t <= 512 ? 4 : (max_t <= 1024 ? 8 : 16); }
+
 bool attention_decode_grouped(int32_t rows, int32_t n_heads, int32_t n_kv, int32_t max_t) {
     if (rows <= 1 || n_kv <= 0 || n_heads % n_kv || n_heads > 32 * 4) return false;
     const int G = n_heads / n_kv, D = n_heads * kHeadDim;
@@ -1080,9 +1101,14 @@ hipError_t launch_attention_decode(hipStream_t s, const float* qkv, int32_t rows
         else if (max_t <= group_max_keys(8))
             TL_KLAUNCH((attention_group_kernel<4, 8>), grid, dim3(512), group_lds_bytes(4, tpad, 8), s, p);
         else TL_KLAUNCH((attention_group_kernel<4, kGW>), grid, dim3(kGW * 64), group_lds_bytes(4, tpad, kGW), s, p);
-    } else if (n_heads % 4 == 0 && D <= kRowQPerThread * kNT) {
+    } else if (n_heads % 4 == 0 && D <= kRowMaxD) {
         const size_t lds = (size_t)tpad * 5 + (tpad / 64) * 4 + 16;
-        TL_KLAUNCH((attention_row_kernel<2>), dim3(n_heads, rows), dim3(256), lds, s, p);
+        const dim3 grid(n_heads, rows);
+        switch (attention_row_waves(max_t)) {
+            case 4: TL_KLAUNCH((attention_row_kernel<2, 4>), grid, dim3(256), lds, s, p); break;
+            case 8: TL_KLAUNCH((attention_row_kernel<2, 8>), grid, dim3(512), lds, s, p); break;
+            default: TL_KLAUNCH((attention_row_kernel<2, 16>), grid, dim3(1024), lds, s, p); break;
+        }
     } else {
         const size_t lds = sizeof(float) * W + (size_t)tpad * 4 + tpad + (tpad / 64) * 4 + 64;
         TL_KLAUNCH((attention_decode_kernel<1, 2, 8, 4>), dim3(n_heads, rows), dim3(256), lds, s, p);
@@ -1100,9 +1126,10 @@ hipError_t launch_embed_step(hipStream_t s, const int32_t* tok_by_seq, const int
 }
 
 hipError_t init_decode_kernels() {
-    hipError_t e = hipFuncSetAttribute((const void*)attention_row_kernel<2>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024);
-    if (e != hipSuccess) return e;
+    hipError_t e;
+    for (const void* fn : {(const void*)attention_row_kernel<2, 4>, (const void*)attention_row_kernel<2, 8>,
+                           (const void*)attention_row_kernel<2, 16>})
+        if ((e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024)) != hipSuccess) return e;
     e = hipFuncSetAttribute((const void*)attention_group_kernel<4, kGW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)group_lds_bytes(4, kGroupMaxKeys, kGW));
     if (e != hipSuccess) return e;

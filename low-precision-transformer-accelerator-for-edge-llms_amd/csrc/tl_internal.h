@@ -319,6 +319,9 @@ struct QkvSums {
 // launch_attention_decode takes the grouped (many-row) kernel for these
 // arguments; the only path that accepts QkvSums
 bool attention_decode_grouped(int32_t rows, int32_t n_heads, int32_t n_kv, int32_t max_t);
+// wavefronts per workgroup of the one-row kernel: two 64-key blocks each in
+// registers up to 2048 keys
+int32_t attention_row_waves(int32_t max_t);
 // out_max (the grouped kernel only): [rows][n_heads] max |output| of each head
 hipError_t launch_attention_decode(hipStream_t s, const float* qkv, int32_t rows, int32_t n_heads, int32_t n_kv,
                                    RowMap rm, const float* cos, const float* sin, KvGeom kv, int32_t layer,

@@ -199,7 +199,7 @@ struct tl_handle {
     bool rows_one_seq = false;            // the rows are one sequence at rows_pos0 + r
     int32_t rows_seq = 0, rows_pos0 = 0;
     bool rows_on_host = false;            // ... and its kernels take them as arguments (row_seq / row_pos unused)
-    std::vector<hipGraphExec_t> graphs;   // captured batch-1 decode step per sequence
+    std::vector<hipGraphExec_t> graphs;   // captured batch-1 decode step, by sequence and context bucket
     std::vector<hipGraphExec_t> batch_graphs;   // captured batched decode step, by batch size and context bucket
 
     bool profiling = false;
@@ -561,7 +561,7 @@ int32_t layer_row1(tl_handle* h, int32_t layer, int32_t max_t) {
     }
     {
         Prof p(h, TL_K_ATTN, (double)c.n_heads * max_t * 128.0 + QKV * 4.0 + D * 4.0);
-        unsigned long long* ts = ts_take(h, TL_K_ATTN, (int64_t)c.n_heads * 4);
+        unsigned long long* ts = ts_take(h, TL_K_ATTN, (int64_t)c.n_heads * attention_row_waves(max_t));
         TL_LAUNCH(h, launch_attention_decode(h->stream, h->qkv, 1, c.n_heads, c.n_kv_heads, rowmap(h), h->rope_cos,
                                              h->rope_sin, h->kv, layer, h->kv_sk, h->kv_sv, h->att, max_t, ts));
     }
@@ -980,12 +980,28 @@ int32_t decode_step1(tl_handle* h, int32_t seq, int32_t max_t) {
     return lm_head_rows(h, h->x, 1, seq, 1);
 }
 
-int32_t decode_graph_launch(tl_handle* h, int32_t seq) {
-    if ((int)h->graphs.size() < h->max_seqs) h->graphs.assign(h->max_seqs, nullptr);
-    if (!h->graphs[seq]) {
-        hipGraph_t g = nullptr;
+// context bounds decode steps are captured for: the attention launch depends
+// on its bound (wavefronts per workgroup; batched: the grouped kernel or not)
+constexpr int kCtxBuckets = 4;
+constexpr int32_t kCtxBound[kCtxBuckets - 1] = {512, 1024, 2048};
+int ctx_bucket(int32_t max_t) {
+    int b = 0;
+    while (b < kCtxBuckets - 1 && max_t > kCtxBound[b]) b++;
+    return b;
+}
+int32_t ctx_bound(const tl_handle* h, int bucket) {
+    return bucket < kCtxBuckets - 1 ? std::min(kCtxBound[bucket], h->cfg.max_pos) : h->cfg.max_pos;
+}
+
+// replay of the captured batch-1 step for a position below max_t (captured on
+// first use for this sequence and context bucket)
+int32_t decode_graph_launch(tl_handle* h, int32_t seq, int32_t max_t) {
+    const int bucket = ctx_bucket(max_t);
+    if (h->graphs.empty()) h->graphs.assign((size_t)h->max_seqs * kCtxBuckets, nullptr);
+    hipGraphExec_t& exec = h->graphs[(size_t)seq * kCtxBuckets + bucket];
+    if (!exec) {
         TL_HIP(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        int32_t r = decode_step1(h, seq, h->cfg.max_pos);
+        int32_t r = decode_step1(h, seq, ctx_bound(h, bucket));
         hipGraph_t cap = nullptr;
         hipError_t e = hipStreamEndCapture(h->stream, &cap);
         if (r) {
@@ -993,14 +1009,13 @@ int32_t decode_graph_launch(tl_handle* h, int32_t seq) {
             return r;
         }
         TL_HIP(h, e);
-        g = cap;
         hipGraphExec_t ex = nullptr;
-        e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
+        e = hipGraphInstantiate(&ex, cap, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(cap);
         TL_HIP(h, e);
-        h->graphs[seq] = ex;
+        exec = ex;
     }
-    TL_HIP(h, hipGraphLaunch(h->graphs[seq], h->stream));
+    TL_HIP(h, hipGraphLaunch(exec, h->stream));
     return TL_OK;
 }
 
@@ -1020,22 +1035,15 @@ int32_t batch_step(tl_handle* h, int32_t n_seqs, int32_t max_t) {
     return lm_head_rows(h, h->x, n_seqs, 0, 1);
 }
 
-// context bounds the batched step is captured for: the attention launch
-// depends on its bound (wavefronts per workgroup, grouped kernel or not)
-constexpr int kCtxBuckets = 4;
-constexpr int32_t kCtxBound[kCtxBuckets - 1] = {512, 1024, 2048};
-
 // replay of the captured batched step for positions below max_t (captured on
 // first use for this batch size and context bucket)
 int32_t batch_graph_launch(tl_handle* h, int32_t n_seqs, int32_t max_t) {
-    int bucket = 0;
-    while (bucket < kCtxBuckets - 1 && max_t > kCtxBound[bucket]) bucket++;
-    const int32_t bound = bucket < kCtxBuckets - 1 ? std::min(kCtxBound[bucket], h->cfg.max_pos) : h->cfg.max_pos;
+    const int bucket = ctx_bucket(max_t);
     if (h->batch_graphs.empty()) h->batch_graphs.resize((size_t)(h->max_seqs + 1) * kCtxBuckets, nullptr);
     hipGraphExec_t& exec = h->batch_graphs[(size_t)n_seqs * kCtxBuckets + bucket];
     if (!exec) {
         TL_HIP(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        int32_t r = batch_step(h, n_seqs, bound);
+        int32_t r = batch_step(h, n_seqs, ctx_bound(h, bucket));
         hipGraph_t cap = nullptr;
         hipError_t e = hipStreamEndCapture(h->stream, &cap);
         if (r) {
@@ -1784,8 +1792,9 @@ int32_t tl_decode(tl_handle* h, int32_t seq, int32_t max_new, int32_t eos_id, co
     if ((r = set_decode_row(h, seq, h->host_cursor[seq], eos_id))) return r;
     if ((r = decode_embed1(h))) return r;
     auto launch_step = [&](int32_t i) -> int32_t {
-        if (!h->profiling) return decode_graph_launch(h, seq);
-        return decode_step1(h, seq, h->host_cursor[seq] + i + 1);   // profiling: direct launches
+        const int32_t keys = h->host_cursor[seq] + i + 1;   // at most: the device stops advancing at EOS
+        if (!h->profiling) return decode_graph_launch(h, seq, keys);
+        return decode_step1(h, seq, keys);   // profiling: direct launches
     };
     volatile int32_t* abort_word = h->ctl_host;
     volatile int32_t* stop_mirror = h->ctl_host + 1 + seq;
@@ -2130,7 +2139,7 @@ int32_t tl_decode_timeline(tl_handle* h, int32_t seq, int32_t n_steps, tl_timeli
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
-        r = decode_step1(h, seq, c.max_pos);
+        r = decode_step1(h, seq, ctx_bound(h, ctx_bucket(h->host_cursor[seq] + n_steps)));
         e = hipStreamEndCapture(h->stream, &graph);
     }
     h->ts_on = false;

@@ -92,3 +92,45 @@ def test_layer_rows_equal_single_rows(layer_eng, rows):
     for g in range(4):
         for a, b in zip(layer_eng.kv_read(0, 0, g, 0, rows), layer_eng.kv_read(1, 0, g, 0, rows)):
             assert_bits_equal(a, b, f"cache head {g}")
+
+
+@pytest.mark.parametrize("pos", [1, 511, 512, 700, 1023, 1024, 1535, 2046])
+def test_single_row_attention_wavefront_counts(layer_eng, pos):
+    """Batch-1 attention at both sides of its context bounds (4, 8 and 16
+    wavefronts): two rows at pos, pos + 1 one by one equal the two rows as one
+    block, which the prefill attention computes."""
+    rng = np.random.default_rng(pos)
+    for g in range(4):
+        k, v = (np.clip(np.rint(rng.standard_normal((pos, 64)) * 25), -127, 127).astype(np.int8) for _ in range(2))
+        layer_eng.kv_write(0, 0, g, 0, k, v)
+        layer_eng.kv_write(1, 0, g, 0, k, v)
+    x = rng.standard_normal((2, oracle.TINYLLAMA_CFG["hidden"])).astype(F32)
+    both, one = dev(x), dev(x)
+    layer_eng.rt.call("tl_layer_rows", 0, 0, pos, 2, both)
+    for r in range(2):
+        layer_eng.decode_layer(one[r], 0, pos + r, seq=1)
+    assert_bits_equal(host(one), host(both), f"rows at {pos}, {pos + 1}")
+    for g in range(4):
+        for a, b in zip(layer_eng.kv_read(0, 0, g, pos, 2), layer_eng.kv_read(1, 0, g, pos, 2)):
+            assert_bits_equal(a, b, f"cache head {g}")
+
+
+@pytest.mark.parametrize("n,new", [(500, 30), (1015, 25)])
+def test_decode_crosses_a_context_bound(n, new):
+    """One decode call whose steps pass 512 or 1024 keys (another captured
+    step from there on) writes the K/V rows that a prefill of the whole
+    sequence writes, and predicts the same next token."""
+    from lpta.engine import Engine
+    eng = Engine(dict(oracle.TINYLLAMA_CFG, n_layers=2, vocab=4096), max_seqs=2)
+    eng.load_random(3)
+    prompt = np.random.default_rng(n).integers(0, 4096, n).astype(np.int32)
+    first, _ = eng.prefill(prompt, seq=0)
+    got, _ = eng.decode(new, seq=0)
+    fed = np.concatenate([prompt, [first], got[:-1]]).astype(np.int32)
+    nxt, _ = eng.prefill(fed, seq=1)
+    assert nxt == got[-1]
+    for layer in range(2):
+        for g in range(4):
+            for a, b in zip(eng.kv_read(0, layer, g, 0, fed.size), eng.kv_read(1, layer, g, 0, fed.size)):
+                assert_bits_equal(a, b, f"layer {layer} head {g}")
+    eng.close()
