@@ -209,7 +209,8 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(AttnDecodeArg
     const int g = h0 / G;
     const int row = blockIdx.y;
     const int D = p.n_heads * kHeadDim, KVD = p.n_kv * kHeadDim, W = D + 2 * KVD;
-    const int pos = p.rm.pos_of(row), seq = p.rm.seq_of(row);
+    int pos, seq;
+    p.rm.get(row, seq, pos);
     if (pos < 0 || pos >= p.kv.max_pos) return;   // a row outside the cache (uniform per workgroup)
     const int T = pos + 1;
     const int tpad = (T + 63) & ~63;
@@ -448,7 +449,8 @@ __global__ __launch_bounds__(NW * 64) void attention_row_kernel(AttnDecodeArgs p
     }
     const int g = h0 / G, row = blockIdx.y;
     const int D = p.n_heads * kHeadDim, KVD = p.n_kv * kHeadDim, W = D + 2 * KVD;
-    const int pos = p.rm.pos_of(row), seq = p.rm.seq_of(row);
+    int pos, seq;
+    p.rm.get(row, seq, pos);
     if (pos < 0 || pos >= p.kv.max_pos) return;   // a row outside the cache (uniform per workgroup)
     const int T = pos + 1, tpad = (T + 63) & ~63, nblk = tpad >> 6;
     const int64_t pl = p.kv.plane(seq, p.layer, g);
@@ -709,7 +711,8 @@ __global__ __launch_bounds__(NWV * 64) void attention_group_kernel(AttnDecodeArg
     }
     const int g = h0 / G;
     const int D = p.n_heads * kHeadDim, KVD = p.n_kv * kHeadDim, W = D + 2 * KVD;
-    const int pos = p.rm.pos_of(row), seq = p.rm.seq_of(row);
+    int pos, seq;
+    p.rm.get(row, seq, pos);
     if (pos < 0 || pos >= p.kv.max_pos) return;   // a row outside the cache (uniform per workgroup)
     const int T = pos + 1, tpad = (T + 63) & ~63, nblk = tpad >> 6;
     const int64_t pl = p.kv.plane(seq, p.layer, g);

@@ -381,6 +381,24 @@ TL_DEV unsigned long long half_max_u64(unsigned long long v) {
     return max_u64(((unsigned long long)ph[0] << 32) | pl[0], ((unsigned long long)ph[1] << 32) | pl[1]);
 }
 
+// the best argmax key of each half-wavefront's 32 logits, lane l holding index
+// base + l % 32 (valid: take part), the same in every lane of the half: the
+// maximum of the keys' upper words, then the lowest lane that has it
+TL_DEV unsigned long long half_argmax_key(float v, bool valid, int32_t base) {
+    const unsigned u = valid ? (unsigned)(argmax_key(v, 0) >> 32) : 0u;
+    unsigned m = u;
+    m = max(m, (unsigned)dpp<kDppXor1>((int)m));
+    m = max(m, (unsigned)dpp<kDppXor2>((int)m));
+    m = max(m, (unsigned)dpp<kDppHalfMirror>((int)m));
+    m = max(m, (unsigned)dpp<kDppRowMirror>((int)m));
+    const auto p = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+    m = max(p[0], p[1]);
+    const unsigned long long eq = __builtin_amdgcn_ballot_w64(u == m && valid);
+    const unsigned half = lane_id() & 32 ? (unsigned)(eq >> 32) : (unsigned)eq;
+    if (half == 0) return 0ull;
+    return ((unsigned long long)m << 32) | (0xFFFFFFFFu - (unsigned)(base + __builtin_ctz(half)));
+}
+
 // 128-bit loads that stay 128-bit: weights stream through once (non-temporal)
 TL_DEV v4i ld_nt16(const int8_t* p) { return __builtin_nontemporal_load((const v4i*)p); }
 TL_DEV v4i ld16(const int8_t* p) { return *(const v4i*)p; }

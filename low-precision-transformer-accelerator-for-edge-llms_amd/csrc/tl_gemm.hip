@@ -491,20 +491,26 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(GemmArgs a) {
                 } else {
                     out = v0;
                 }
+                if constexpr (EPI == EPI_ARGMAX) {
+                    // the best key of row m over the block's 32 columns, the lanes of
+                    // a half-wavefront (argmax_tiles_kernel folds the blocks)
+                    const unsigned long long key = half_argmax_key(out, n < a.n, n - (lane & 31));
+                    if ((lane & 31) == 0 && m < a.m && n < a.n) a.key[(int64_t)(n >> 5) * a.m + m] = key;
+                    continue;
+                }
                 if (m < a.m && n < a.n) a.y[(int64_t)m * a.n + n] = out;
             }
         }
 }
 
-// Row-major operands (the tl_gemm_i8 operator, and prefill shapes the packed
-// path does not take), M >= 64, 32x32x32 MFMA tiles:
+// Row-major operands (the tl_gemm_i8 operators, the LM head over many rows and
+// prefill shapes the packed path does not take), M >= 64, 32x32x32 MFMA tiles:
 //   gemm_tile_kernel, K a multiple of 128: 2 x 2 wavefronts of one 32 x 32
 //     block each (64 x 64 block tile), 128-byte K stages through two LDS
-//     buffers, four register sets;
+//     buffers, four register sets; or of 2 x 2 blocks each (128 x 128 block
+//     tile, 64-byte stages, two register sets) where tile_large says so;
 //   gemm32_kernel otherwise: 2 x 2 x 2 wavefronts (the K slice split in two
 //     inside the workgroup), 64 x 64 block tile, three register sets.
-// At M = 512 the 64 x 64 tiles measured fastest; larger block tiles leave CUs
-// idle at these N.
 template <int WM, int WN, int TM, int TN, int BK, int PD, int KS, int EPI>
 static void go32(hipStream_t s, const GemmArgs& a, int32_t splits) {
     using G = GemmShape<WM, WN, TM, TN, BK, PD, KS>;
@@ -521,8 +527,23 @@ static bool go_tile(hipStream_t s, const GemmArgs& a) {
     return true;
 }
 
+// 128 x 128 tiles read half of the LDS bytes per product but come in a quarter
+// of the number: they win where the 64 x 64 tiles need at least three rounds of 256
+// for each of theirs (K = 2048, N x M: 2048 x 2048 17.3 us against 20.8, 5632 x
+// 2048 38.7 against 47.6, 5632 x 1000 25.5 against 27.3, 32000 x 512 60 against
+// 90; 2560 x 1000, at the line, 16.0 against 15.9; below it 2560 x 2048 25.3
+// against 24.5, 2048 x 1000 14.8 against 11.9).
+static bool tile_large(int64_t m, int64_t n) {
+    const int64_t r64 = (((n + 63) / 64) * ((m + 63) / 64) + 255) / 256;
+    const int64_t r128 = (((n + 127) / 128) * ((m + 127) / 128) + 255) / 256;
+    return r64 >= 3 * r128;
+}
+
 template <int EPI>
 static bool shape32(hipStream_t s, const GemmArgs& a, bool tile) {
+    if constexpr (EPI != EPI_GLU)
+        if (tile && tile_large(a.m, a.n)) return go_tile<2, 2, 2, 2, 64, 2, EPI>(s, a);
+    if constexpr (EPI == EPI_ARGMAX) return go_tile<2, 2, 1, 1, 128, 4, EPI>(s, a);   // tile only (launch_gemm32)
     if (tile) return go_tile<2, 2, 1, 1, 128, 4, EPI>(s, a);
     go32<2, 2, 1, 1, 128, 3, 2, EPI>(s, a, 1);
     return true;
@@ -541,6 +562,7 @@ hipError_t launch_gemm32(hipStream_t s, int epi, const GemmArgs& args, bool tile
         case EPI_DEQUANT_RES: ok = shape32<EPI_DEQUANT_RES>(s, a, tile); break;
         case EPI_GLU: ok = shape32<EPI_GLU>(s, a, tile); break;
         case EPI_RAW: ok = shape32<EPI_RAW>(s, a, tile); break;
+        case EPI_ARGMAX: ok = tile && a.key && shape32<EPI_ARGMAX>(s, a, tile); break;
         default: break;
     }
     if (!ok) return hipErrorInvalidValue;
@@ -632,8 +654,7 @@ TL_DEV void qkv_rope_operands(const GemmArgs& a, const QkvRopeArgs& f, int mt0, 
     for (int ee = 0; ee < NE; ee++) {
         const int e = o.e0 + ee, m = min(o.rb + 8 * (e >> 2) + (e & 3), a.m - 1);
         o.sx[ee] = a.as[m];
-        o.pos[ee] = f.rm.pos_of(m);
-        o.seq[ee] = f.rm.seq_of(m);
+        f.rm.get(m, o.seq[ee], o.pos[ee]);
     }
 }
 
@@ -820,13 +841,6 @@ __global__ __launch_bounds__(256) void gemm_pk_split_kernel(GemmArgs a, QkvRopeA
         for (int e = 0; e < 16; e++) {
             const int m = rb + 8 * (e >> 2) + (e & 3);
             const float v = (float)sum[e] * deq_mult(so.sx[bw][e], so.sw[bw]);
-            if constexpr (EPI == EPI_ARGMAX) {
-                // the best key of row m over the block's 32 columns (the
-                // lanes of a half-wavefront), as gemm_rows32_kernel's
-                const unsigned long long k = half_max_u64(argmax_key(v, n));
-                if ((lane & 31) == 0 && m < a.m) a.key[(int64_t)(nt0 + j) * a.m + m] = k;
-                continue;
-            }
             if (m < a.m) a.y[(int64_t)m * a.n + n] = RES ? so.res[bw][RES ? e : 0] + v : v;
         }
     }
@@ -995,7 +1009,6 @@ static bool pk_split_narrow(int32_t m, int32_t n) {
 bool gemm_pk_supported(int epi, int32_t m, int32_t n, int32_t k) {
     if (m < 1 || n < 1 || k < 1) return false;
     if (epi == EPI_GLU) return n % 64 == 0 && k % 256 == 0;   // both tile widths
-    if (epi == EPI_ARGMAX) return n % 64 == 0 && k % 512 == 0;
     if (epi != EPI_DEQUANT && epi != EPI_DEQUANT_RES) return false;
     return k % 512 == 0 && (n % 64 == 0 || pk_split_narrow(m, n));
 }
@@ -1010,12 +1023,6 @@ hipError_t launch_gemm_pk(hipStream_t s, int epi, const GemmArgs& a) {
     const QkvRopeArgs f{};
     if (epi == EPI_GLU) {
         TL_KLAUNCH(gemm_pk_glu_kernel<1>, dim3(a.n / 32, (a.m + 127) / 128), block, pk_glu_lds_bytes(1), s, a);
-        return hipGetLastError();
-    }
-    if (epi == EPI_ARGMAX) {
-        if (!a.key) return hipErrorInvalidValue;
-        TL_KLAUNCH((gemm_pk_split_kernel<2, 2, EPI_ARGMAX>), dim3(a.n / 64, (a.m + 63) / 64), block,
-                   pk_split_lds_bytes(2, 2), s, a, f);
         return hipGetLastError();
     }
     const bool res = epi == EPI_DEQUANT_RES;
@@ -1047,12 +1054,10 @@ hipError_t init_gemm_pk_kernels() {
                          (const void*)gemm_pk_split_kernel<1, 5, EPI_DEQUANT_RES>,
                          (const void*)gemm_pk_split_kernel<2, 2, EPI_DEQUANT>,
                          (const void*)gemm_pk_split_kernel<2, 2, EPI_DEQUANT_RES>, (const void*)gemm_pk_glu_kernel<1>,
-                         (const void*)gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>,
-                         (const void*)gemm_pk_split_kernel<2, 2, EPI_ARGMAX>};
+                         (const void*)gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>};
     const size_t bytes[] = {pk_split_lds_bytes(1, 5), pk_split_lds_bytes(1, 5), pk_split_lds_bytes(2, 2),
-                            pk_split_lds_bytes(2, 2), pk_glu_lds_bytes(1), pk_split_lds_bytes(2, 2),
-                            pk_split_lds_bytes(2, 2)};
-    for (int i = 0; i < 7; i++) {
+                            pk_split_lds_bytes(2, 2), pk_glu_lds_bytes(1), pk_split_lds_bytes(2, 2)};
+    for (int i = 0; i < 6; i++) {
         const hipError_t e = hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes[i]);
         if (e != hipSuccess) return e;
     }

@@ -52,8 +52,15 @@ struct RowMap {
     const int32_t* seq;  // [rows] sequence (KV plane) of each row, or null: seq0
     const int32_t* pos;  // [rows] position of each row, or null: pos0 + row
     int32_t seq0, pos0;
-    __host__ __device__ int32_t seq_of(int32_t row) const { return seq ? seq[row] : seq0; }
-    __host__ __device__ int32_t pos_of(int32_t row) const { return pos ? pos[row] : pos0 + row; }
+    __host__ __device__ void get(int32_t row, int32_t& s, int32_t& p) const {
+        if (pos) {   // both loads in flight together
+            s = seq[row];
+            p = pos[row];
+        } else {
+            s = seq0;
+            p = pos0 + row;
+        }
+    }
 };
 
 enum GemvEpi : int {
@@ -114,7 +121,7 @@ struct GemmArgs {
     int32_t k_split;          // K elements per split (multiple of 64; gemm_rows32: multiple of 32, 0 = K)
     const int8_t* wp;         // packed copy of w (MFMA operand blocks, pack_weights_kernel) or null
     const int8_t* wp2;        // packed copy of w2
-    unsigned long long* key;  // EPI_ARGMAX: [N / 32 tiles][M] best key of each tile and row
+    unsigned long long* key;  // EPI_ARGMAX: [N / 32][M] best key of each 32 columns and row
     const int8_t* ap;         // A in MFMA operand blocks (rows padded to gemm_pk_row_pad()) for
                               // launch_gemm_pk, or null
     // gemm_rows32 EPI_ACC_F32 only: A is the float32 [M][K] row-major

@@ -729,7 +729,8 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(const float* __restrict__
     const float4* src = (const float4*)(qkv + (int64_t)row * W);
     for (int c = tid; c < W / 4; c += blockDim.x) ((float4*)v)[c] = src[c];
     __syncthreads();
-    const int pos = rm.pos_of(row), seq = rm.seq_of(row);
+    int pos, seq;
+    rm.get(row, seq, pos);
     if (pos < 0 || pos >= kv.max_pos) return;   // a row outside the cache (uniform per workgroup)
     const float* cp = cosb + (int64_t)pos * kHeadDim;
     const float* sp = sinb + (int64_t)pos * kHeadDim;
@@ -799,7 +800,8 @@ __global__ __launch_bounds__(256) void attention_kernel(const int8_t* __restrict
     const int g = blockIdx.x, row = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int G = n_heads / n_kv;
-    const int pos = rm.pos_of(row), seq = rm.seq_of(row);
+    int pos, seq;
+    rm.get(row, seq, pos);
     if (pos < 0 || pos >= kv.max_pos) return;   // a row outside the cache (uniform per workgroup)
     const int T = pos + 1;
     const int tpad = (T + 63) & ~63;

@@ -853,7 +853,8 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
         Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + D * 8.0);
         TL_LAUNCH(h, launch_gemv_fused(h->stream, PRO_RMSNORM, EPI_ARGMAX, g));
     } else {
-        const bool lm_pk = rows > 32 && h->lm_wp && h->plan.n_leaves <= 64 && gemm_pk_supported(EPI_ARGMAX, rows, V, D);
+        // past 32 rows: row-major tiles with the argmax in their epilogue
+        const bool lm_tile = rows > 32 && D % 128 == 0 && V % 32 == 0;
         if (h->racc_res_ws && xrow == h->x) {
             int32_t r = rows_rmsnorm(h, rows, h->g_final);
             if (r) return r;
@@ -861,14 +862,13 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
             int32_t r = discard_pending_sums(h);
             if (r) return r;
             Prof p(h, TL_K_NORM, (double)rows * D * 9.0);
-            TL_LAUNCH(h, launch_rmsnorm_quant(h->stream, xrow, h->g_final, rows, D, c.rms_eps, h->plan, nullptr, h->a8, h->as, lm_pk));
+            TL_LAUNCH(h, launch_rmsnorm_quant(h->stream, xrow, h->g_final, rows, D, c.rms_eps, h->plan, nullptr, h->a8, h->as));
         }
         GemmArgs a{};
-        if (lm_pk) a.ap = h->a8;
         a.a = h->a8; a.w = h->lm_w; a.as = h->as; a.ws = h->lm_s; a.y = h->logits; a.m = rows; a.n = V; a.k = D;
-        if (lm_pk || (rows <= 32 && h->lm_wp && D % 64 == 0 && D <= 2048)) {
-            // packed-weight MFMA GEMM with the argmax in its epilogue (one key
-            // per 32-column tile and row), then the tiles' keys folded per row
+        if (lm_tile || (rows <= 32 && h->lm_wp && D % 64 == 0 && D <= 2048)) {
+            // MFMA GEMM (up to 32 rows on the packed weights) with the argmax in its
+            // epilogue, one key per 32 columns and row, then these keys folded per row
             const int tiles = V / 32;
             int32_t r = ensure_partials(h, (size_t)tiles * rows * 2);
             if (r) return r;
@@ -876,7 +876,7 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
             a.key = (unsigned long long*)h->partials;
             a.y = nullptr;
             Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + (double)rows * D);
-            if (lm_pk) TL_LAUNCH(h, launch_gemm_pk(h->stream, EPI_ARGMAX, a));
+            if (lm_tile) TL_LAUNCH(h, launch_gemm32(h->stream, EPI_ARGMAX, a, true));
             else TL_LAUNCH(h, launch_gemm_rows32(h->stream, EPI_ARGMAX, a, rows32_waves(EPI_ARGMAX)));
             TL_LAUNCH(h, launch_argmax_tiles(h->stream, a.key, tiles, rows, keys));
         } else {
