@@ -711,8 +711,7 @@ __global__ __launch_bounds__(NWV * 64) void attention_group_kernel(AttnDecodeArg
     }
     const int g = h0 / G;
     const int D = p.n_heads * kHeadDim, KVD = p.n_kv * kHeadDim, W = D + 2 * KVD;
-    int pos, seq;
-    p.rm.get(row, seq, pos);
+    const int pos = p.rm.pos[row], seq = p.rm.seq[row];   // rows of a batch: always the arrays
     if (pos < 0 || pos >= p.kv.max_pos) return;   // a row outside the cache (uniform per workgroup)
     const int T = pos + 1, tpad = (T + 63) & ~63, nblk = tpad >> 6;
     const int64_t pl = p.kv.plane(seq, p.layer, g);
@@ -1083,6 +1082,7 @@ hipError_t launch_attention_decode(hipStream_t s, const float* qkv, int32_t rows
                      nullptr, nullptr, nullptr, nullptr};
     const bool grouped = attention_decode_grouped(rows, n_heads, n_kv, max_t);
     if (out_max && !grouped) return hipErrorInvalidValue;
+    if (grouped && (!rm.seq || !rm.pos)) return hipErrorInvalidValue;
     p.out_max = out_max;
     if (sums) {
         if (!grouped || !sums->acc || !sums->as || !sums->ws) return hipErrorInvalidValue;
