@@ -528,15 +528,16 @@ static bool go_tile(hipStream_t s, const GemmArgs& a) {
 }
 
 // 128 x 128 tiles read half of the LDS bytes per product but come in a quarter
-// of the number: they win where the 64 x 64 tiles need at least three rounds of 256
-// for each of theirs (K = 2048, N x M: 2048 x 2048 17.3 us against 20.8, 5632 x
-// 2048 38.7 against 47.6, 5632 x 1000 25.5 against 27.3, 32000 x 512 60 against
-// 90; 2560 x 1000, at the line, 16.0 against 15.9; below it 2560 x 2048 25.3
-// against 24.5, 2048 x 1000 14.8 against 11.9).
+// of the number: they win where the 64 x 64 tiles need at least four rounds of 256,
+// and three for each of theirs (K = 2048, N x M, whole calls: 2048 x 1600 30.8 us against
+// 34.0, 2560 x 1400 30.6 against 33.7, 5632 x 600 30.4 against 33.6, 5632 x 2048
+// 51.9 against 60.1, and the kernel at 32000 x 512 60 against 90; outside, 2560 x
+// 820, three rounds against one, 29.5 against 29.0, 2048 x 1280 30.6 against 30.0,
+// 5632 x 769, five against two, 38.4 against 36.5).
 static bool tile_large(int64_t m, int64_t n) {
     const int64_t r64 = (((n + 63) / 64) * ((m + 63) / 64) + 255) / 256;
     const int64_t r128 = (((n + 127) / 128) * ((m + 127) / 128) + 255) / 256;
-    return r64 >= 3 * r128;
+    return r64 >= 4 && r64 >= 3 * r128;
 }
 
 template <int EPI>

@@ -20,9 +20,11 @@ def rt():
 
 @pytest.mark.parametrize("m,n,k", [
     (2048, 2048, 128),    # 128 x 128 tiles, one round, two 64-byte stages
-    (1999, 2081, 256),    # ... ragged rows and columns
+    (1999, 2017, 256),    # ... ragged rows and columns
+    (1999, 2081, 256),    # five rounds of 64 x 64 tiles against two: 64 x 64, ragged
     (65, 32000, 128),     # ... the second row half of every tile nearly empty
     (2048, 2560, 384),    # just below the rule: 64 x 64 tiles
+    (1100, 2048, 128),    # three rounds against one: 64 x 64
     (333, 9000, 1152),
     (64, 64, 128),
 ])
