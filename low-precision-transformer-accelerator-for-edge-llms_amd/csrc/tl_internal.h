@@ -175,8 +175,9 @@ struct FoldArgs {
     int32_t rows, n;
     float eps;
     PwPlan plan;
-    int8_t* q;            // [rows][n]
+    int8_t* q;            // [rows][n], or with packed the operand blocks of launch_gemm_pk
     double* scales;       // [rows]
+    int32_t packed;
     int32_t* zero;        // or null: [rows][zero_n] int32 the kernel also clears (consumed integer sums)
     int32_t zero_n;
     L2Prefetch pf;        // the next GEMM's weight tiles (pf.w[0] null: none)

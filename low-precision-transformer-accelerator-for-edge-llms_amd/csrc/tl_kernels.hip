@@ -244,8 +244,14 @@ __global__ __launch_bounds__(kNT) void rows_fold_kernel(FoldArgs f) {
         }
     }
     prologue_rmsnorm<KCH>(xv, gv, n, f.eps, f.plan, sq, part, xs8, red, &xscale);
-    int8_t* qr = f.q + ro;
-    for (int o = tid * 16; o < n; o += kNT * 16) *(v4i*)(qr + o) = *(const v4i*)(xs8 + o);
+    if (f.packed) {
+        int8_t* qt = f.q + (int64_t)(row >> 5) * (n >> 5) * 1024 + (row & 31) * 16;
+        for (int o = tid * 16; o < n; o += kNT * 16)
+            *(v4i*)(qt + (o >> 5) * 1024 + ((o >> 4) & 1) * 512) = *(const v4i*)(xs8 + o);
+    } else {
+        int8_t* qr = f.q + ro;
+        for (int o = tid * 16; o < n; o += kNT * 16) *(v4i*)(qr + o) = *(const v4i*)(xs8 + o);
+    }
     if (tid == 0) f.scales[row] = xscale;
     if (f.zero)
         for (int i = tid * 4; i < f.zero_n; i += kNT * 4) *(v4i*)(f.zero + (int64_t)row * f.zero_n + i) = (v4i){0, 0, 0, 0};

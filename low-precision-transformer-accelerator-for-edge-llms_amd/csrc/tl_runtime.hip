@@ -604,7 +604,7 @@ static int32_t kslice_len(int32_t n, int32_t k) {
     return ((kch + s - 1) / s) * 32;
 }
 
-// batched decode can run its down GEMM K-sliced
+// 2 to 32 rows on the packed copies, the down GEMM K-sliced where its sums are folded
 static bool kslice_ok(tl_handle* h, const LayerDev& L, int32_t rows) {
     const int D = h->D, F = h->F;
     return h->batch_kslice && rows > 1 && rows <= 32 && L.wd_p && D % 64 == 0 &&
@@ -672,6 +672,7 @@ static int32_t rows_rmsnorm(tl_handle* h, int32_t rows, const float* g, bool pk 
         FoldArgs f{};
         f.x = h->x; f.acc = h->racc; f.as = h->as; f.ws = h->racc_res_ws; f.g = g;
         f.rows = rows; f.n = h->D; f.eps = h->cfg.rms_eps; f.plan = h->plan; f.q = h->a8; f.scales = h->as;
+        f.packed = pk;
         if (pf) f.pf = *pf;
         h->racc_res_ws = nullptr;
         {
@@ -691,14 +692,24 @@ static int32_t rows_rmsnorm(tl_handle* h, int32_t rows, const float* g, bool pk 
 // position are in h->row_seq / h->row_pos; max_t bounds pos + 1 over the rows.
 // decode: every row is a different sequence (its own K/V row is appended by
 // the attention kernel); otherwise the rows are consecutive prompt positions
-// of one sequence (all appended before attention reads them).
-int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, bool decode) {
+// of one sequence (all appended before attention reads them).  The caller has
+// discarded pending sums (discard_pending_sums) before the first layer.  chain:
+// another rows_rmsnorm of h->x follows (the next layer's, or a batch's final one);
+// without it the layer leaves h->x complete.
+int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, bool decode, bool chain) {
     if (rows == 1) return layer_row1(h, layer, max_t);
     const tl_config& c = h->cfg;
     const LayerDev& L = h->layers[layer];
     const int D = h->D, F = h->F, KVD = h->KVD, QKV = h->QKV;
-    const bool ks = decode && kslice_ok(h, L, rows);
-    const bool qks = ks && qkv_kslice_ok(h, L, rows, max_t);
+    // up to 32 rows of a batch or a prompt: the row kernels prefetch the next
+    // GEMM's weight tiles, with a row kernel to fold it the down GEMM is
+    // K-sliced, and a prompt's Q|K|V GEMM does qkv_post's work (fq), one launch
+    // less: one layer over 5 rows 88 -> 77 us, 32 rows 104 -> 87 us, 22 layers and the
+    // head over 20 rows 1.38 -> 1.26 ms, 32 rows 1.54 -> 1.30 ms (K slices
+    // and the head on packed weights give most of the latter two)
+    const bool few = kslice_ok(h, L, rows);
+    const bool ks = few && chain;
+    const bool qks = ks && decode && qkv_kslice_ok(h, L, rows, max_t);
     // the O GEMM K-sliced with the attention output quantized in it (one
     // 32-byte K chunk per wavefront of the 16-wavefront small-M GEMM)
     const bool of = qks && h->o_fuse && L.wo_p && c.n_heads <= 32 && c.n_heads % 4 == 0 &&
@@ -706,8 +717,9 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
     const bool pk = (!decode || rows > 32) && prefill_packed(h, L, rows);   // h->a8 in the packed GEMM operand layout
     // prefill tiles on packed operands: qkv_post's work in the Q|K|V GEMM
     // epilogue, rotated Q in h->qkv ([rows][D]) quantized by the attention tiles
-    const bool fq = pk && h->rows_one_seq && h->rows_pos0 + rows <= kTileMaxKeys && D % 64 == 0 &&
-                    KVD % 64 == 0;
+    // (up to 32 rows only the operand of that GEMM is packed)
+    const bool fq = (pk || (few && !decode && L.wqkv_p && gemm_pk_supported(EPI_DEQUANT, rows, QKV, D))) &&
+                    h->rows_one_seq && h->rows_pos0 + rows <= kTileMaxKeys && D % 64 == 0 && KVD % 64 == 0;
     // The row kernel before a GEMM also brings that GEMM's packed weight tiles
     // into the L2 of the XCD whose workgroups read them: the packed GEMMs'
     // grids have a multiple of 8 column tiles in x, so column tile t runs on
@@ -724,15 +736,14 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
         p.sink = h->pf_sink;
         return p;
     };
-    const bool l2pf = ks || pk;
+    const bool l2pf = few || pk;
     auto tc = [&](int n, int k) { return pk && !pk_rows32(EPI_DEQUANT, rows, n, k) ? 64 : 32; };
     const bool q32 = pk && !fq && pk_rows32(EPI_DEQUANT, rows, QKV, D);
     const L2Prefetch pf_qkv = pf_plan(L.wqkv_p, nullptr, 1, fq ? 64 : 32, QKV, D), pf_o = pf_plan(L.wo_p, nullptr, 1, tc(D, D), D, D),
                      pf_glu = pf_plan(L.wg_p, L.wu_p, 2, 32, F, D), pf_down = pf_plan(L.wd_p, nullptr, 1, tc(D, F), D, F);
-    const L2Prefetch* pfq = l2pf && (ks || fq || q32) ? &pf_qkv : nullptr;   // prefill: the RoPE-epilogue tiles
+    const L2Prefetch* pfq = l2pf && (few || fq || q32) ? &pf_qkv : nullptr;   // prefill: the RoPE-epilogue tiles
     int32_t r;
-    if (!ks && (r = discard_pending_sums(h))) return r;
-    if ((r = rows_rmsnorm(h, rows, L.g_in, pk, pfq))) return r;
+    if ((r = rows_rmsnorm(h, rows, L.g_in, pk || fq, pfq))) return r;
     if (qks) {
         // Q|K|V (K = D) K-sliced over the chip: the attention kernel
         // dequantizes the integer sums it reads from h->qacc
@@ -800,7 +811,7 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
             Prof p(h, TL_K_NORM, (double)rows * D * 5.0 + (qks ? (double)rows * QKV * 4.0 : 0.0));
             TL_LAUNCH(h, launch_quantize_rows(h->stream, h->att, rows, D, h->a8, h->as, zero,
                                               qks ? QKV : (fq ? kQmaxStride : 0), pk,
-                                              l2pf && pk ? &pf_o : nullptr));
+                                              l2pf ? &pf_o : nullptr));
             if (qks) h->qacc_clean = true;
             if (fq) h->qmax_clean = true;
         }
@@ -1031,7 +1042,7 @@ int32_t batch_step(tl_handle* h, int32_t n_seqs, int32_t max_t) {
     TL_LAUNCH(h, launch_embed_step(h->stream, h->token_cur, h->row_seq, n_seqs, h->cursor, h->row_pos, h->D, c.vocab,
                                    h->emb, h->emb_s, h->x));
     for (int l = 0; l < c.n_layers; l++)
-        if ((r = layer_rows(h, l, n_seqs, max_t, true))) return r;
+        if ((r = layer_rows(h, l, n_seqs, max_t, true, true))) return r;
     return lm_head_rows(h, h->x, n_seqs, 0, 1);
 }
 
@@ -1138,7 +1149,7 @@ int32_t tl_create(const tl_config* cfg, int32_t max_seqs, tl_handle** out) {
         (e = dalloc(h, &h->token_cur, (size_t)max_seqs)) || (e = dalloc(h, &h->cursor, (size_t)max_seqs)) ||
         (e = dalloc(h, &h->n_gen, (size_t)max_seqs)) || (e = dalloc(h, &h->eos_id, (size_t)max_seqs)) ||
         (e = dalloc(h, &h->stopped, (size_t)max_seqs)) ||
-        (e = dalloc(h, &h->racc, h->racc_cap = (size_t)std::min(32, max_seqs) * D)) ||
+        (e = dalloc(h, &h->racc, h->racc_cap = (size_t)std::min(32, h->max_rows) * D)) ||
         (e = dalloc(h, &h->qacc, h->qacc_cap = (size_t)std::min(32, max_seqs) * h->QKV)) ||
         (e = dalloc(h, &h->pf_sink, 1)) ||
         (e = dalloc(h, &h->qmax, (size_t)kQmaxStride * R)) ||
@@ -1654,7 +1665,7 @@ int32_t tl_decode_layer(tl_handle* h, int32_t seq, int32_t layer, int32_t pos, f
     set_rows(h, seq, pos);
     const CallerRows cx(h, x, 1);
     TL_HIP(h, cx.in());
-    if ((r = layer_rows(h, layer, 1, pos + 1, true))) return r;
+    if ((r = layer_rows(h, layer, 1, pos + 1, true, false))) return r;
     TL_HIP(h, cx.out());
     return finish(h);
 }
@@ -1688,6 +1699,7 @@ int32_t prefill_layers(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t
     init.stopped = h->stopped + seq;
     TL_LAUNCH(h, launch_rows_init(h->stream, init));
     TL_LAUNCH(h, launch_embed(h->stream, h->tokens, n, h->D, h->cfg.vocab, h->emb, h->emb_s, h->x));
+    if ((r = discard_pending_sums(h))) return r;
     for (int l = 0; l < c.n_layers; l++) {
         if (abort_flag) {
             if (l > 0) {
@@ -1704,7 +1716,7 @@ int32_t prefill_layers(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t
                 return finish(h);
             }
         }
-        if ((r = layer_rows(h, l, n, n, false))) return r;
+        if ((r = layer_rows(h, l, n, n, false, l + 1 < c.n_layers))) return r;
         if (abort_flag) TL_HIP(h, hipEventRecord(h->watch_ev[0], h->stream));
     }
     return TL_OK;
@@ -1746,6 +1758,7 @@ int32_t tl_prefill_logits(tl_handle* h, int32_t seq, const int32_t* tokens, int3
     }
     GemmArgs a{};
     a.a = h->a8; a.w = h->lm_w; a.as = h->as; a.ws = h->lm_s; a.y = logits; a.m = n; a.n = c.vocab; a.k = h->D;
+    a.wp = h->lm_wp;
     if ((r = run_gemm(h, EPI_DEQUANT, a, TL_K_LMHEAD))) return r;
     return prefill_finish(h, seq, n, nullptr, nullptr);
 }
@@ -1762,7 +1775,8 @@ int32_t tl_layer_rows(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, in
     set_rows(h, seq, pos0);
     const CallerRows cx(h, x, rows);
     TL_HIP(h, cx.in());
-    if ((r = layer_rows(h, layer, rows, pos0 + rows, rows == 1))) return r;
+    if (rows > 1 && (r = discard_pending_sums(h))) return r;
+    if ((r = layer_rows(h, layer, rows, pos0 + rows, rows == 1, false))) return r;
     TL_HIP(h, cx.out());
     return finish(h);
 }

@@ -134,3 +134,39 @@ def test_decode_crosses_a_context_bound(n, new):
             for a, b in zip(eng.kv_read(0, layer, g, 0, fed.size), eng.kv_read(1, layer, g, 0, fed.size)):
                 assert_bits_equal(a, b, f"layer {layer} head {g}")
     eng.close()
+
+
+@pytest.mark.parametrize("n", [2, 5, 31, 32, 33])
+def test_short_prompt_chains_layers(n):
+    """Prompts of up to 32 rows leave each layer's down projection as integer sums that the next layer's RMSNorm
+    folds, and the last layer's complete: the logits of every position, the caches of all layers and a single-layer
+    call after the prompt equal the oracle's."""
+    from lpta.engine import Engine
+    cfg = dict(oracle.TINYLLAMA_CFG, n_layers=3, vocab=512)
+    m = oracle.synthetic_model(cfg, seed=500 + n)
+    eng = Engine(m.cfg, max_seqs=1).load_model(m)
+    orc = oracle.Oracle(m)
+    rng = np.random.default_rng(n)
+    toks = rng.integers(0, cfg["vocab"], n).astype(np.int32)
+    kc, vc = m.new_cache()
+    want = []
+    for p, t in enumerate(toks):
+        x = orc.embed(int(t)).astype(F32)
+        for layer in range(cfg["n_layers"]):
+            x = orc.decode_row(layer, p, x, kc, vc)
+        want.append(np.asarray(orc.lm_head(x, want_logits=True)[2], F32))
+    logits = dev(np.zeros((n, cfg["vocab"]), F32))
+    for _ in range(2):   # the second call finds no sums of the first
+        eng.rt.call("tl_prefill_logits", 0, toks, n, logits)
+        assert_bits_equal(host(logits), np.stack(want), f"logits of {n} positions")
+    for layer in range(cfg["n_layers"]):
+        for g in range(cfg["n_kv_heads"]):
+            k, v = eng.kv_read(0, layer, g, 0, n)
+            assert_bits_equal(k, kc[layer, g, :n], f"K layer {layer} head {g}")
+            assert_bits_equal(v, vc[layer, g, :n], f"V layer {layer} head {g}")
+    x = rng.standard_normal((2, cfg["hidden"])).astype(F32)
+    xs = dev(x)
+    eng.rt.call("tl_layer_rows", 0, 1, n, 2, xs)
+    rows = [orc.decode_row(1, n + r, x[r].copy(), kc, vc) for r in range(2)]
+    assert_bits_equal(host(xs), np.stack(rows), "two rows through one layer")
+    eng.close()
