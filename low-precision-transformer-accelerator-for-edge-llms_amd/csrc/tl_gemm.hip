@@ -619,31 +619,32 @@ TL_DEV void pk_wait_regs(v4i* r) {
 // loads, so they arrive during the last MFMAs.
 constexpr int kPkSplitPD = 4;
 
-static size_t pk_split_lds_bytes(int tm, int tn) { return (size_t)4 * tm * tn * 16 * 64 * sizeof(int); }
+static size_t pk_split_lds_bytes(int tm, int tn, int nwv = 4) { return (size_t)nwv * tm * tn * 16 * 64 * sizeof(int); }
 
-// EPI_QKV_ROPE epilogue of a 64 x 64 tile (one head of Q, K or V): wavefront
-// w takes accumulator registers 8 (w % 2) .. 8 (w % 2) + 7 (8 rows per lane) of
-// row block w / 2 in both column blocks, so a lane holds dimensions d and
-// d + 32 of its rows.  The
+// EPI_QKV_ROPE epilogue of a 32 TM x 64 tile (one head of Q, K or V): wavefront
+// w takes NE = 16 TM / NWV accumulator registers (rows per lane) of one row
+// block in both column blocks, so a lane holds dimensions d and d + 32 of its
+// rows.  The
 // arithmetic is qkv_post_kernel's: x = f32(acc) f32(sx sw), rotated
 // x_d c_d + (-x_{d+32}) s_d and x_{d+32} c_{d+32} + x_d s_{d+32} (two products
 // and a sum, no fused multiply-add), K and V bytes sat(rne(x / s)).  Its
 // operands (row scales, positions, sequences, cos / sin) are loaded before
 // the LDS reduction (qkv_rope_operands, qkv_rope_tables).
-struct QkvRopeOps {   // the 8 registers (rows) of the wavefront's row block
-    double sx[8];
-    int pos[8], seq[8];
-    float c0[8], s0[8], c1[8], s1[8];
+template <int NE>
+struct QkvRopeOps {   // the NE registers (rows) of the wavefront's row block
+    double sx[NE];
+    int pos[NE], seq[NE];
+    float c0[NE], s0[NE], c1[NE], s1[NE];
     float sw0, sw1, sc;
     int region, g, n0, rb, e0, i;
 };
 
+template <int NE>
 TL_DEV void qkv_rope_operands(const GemmArgs& a, const QkvRopeArgs& f, int mt0, int nt0, int wave, int lane,
-                              QkvRopeOps& o) {
-    constexpr int NE = 8;
+                              QkvRopeOps<NE>& o) {
     const int d = lane & 31, D = f.n_heads * kHeadDim, KVD = f.n_kv * kHeadDim;
-    o.i = wave >> 1;
-    o.e0 = (wave & 1) * 8;
+    o.i = wave / (16 / NE);
+    o.e0 = wave % (16 / NE) * NE;
     o.n0 = nt0 * 32;
     o.region = o.n0 < D ? 0 : (o.n0 < D + KVD ? 1 : 2);   // Q, K, V (uniform)
     o.g = o.region == 1 ? (o.n0 - D) >> 6 : (o.n0 - D - KVD) >> 6;
@@ -660,8 +661,8 @@ TL_DEV void qkv_rope_operands(const GemmArgs& a, const QkvRopeArgs& f, int mt0, 
 }
 
 // the cos / sin entries of the rows' positions (after qkv_rope_operands)
-TL_DEV void qkv_rope_tables(const QkvRopeArgs& f, int lane, QkvRopeOps& o) {
-    constexpr int NE = 8;
+template <int NE>
+TL_DEV void qkv_rope_tables(const QkvRopeArgs& f, int lane, QkvRopeOps<NE>& o) {
     const int d = lane & 31;
     if (o.region != 2) {
 #pragma unroll
@@ -675,9 +676,9 @@ TL_DEV void qkv_rope_tables(const QkvRopeArgs& f, int lane, QkvRopeOps& o) {
     }
 }
 
-TL_DEV void qkv_rope_epilogue(const GemmArgs& a, const QkvRopeArgs& f, const QkvRopeOps& o, const int* red,
+template <int NE, int NBLK, int NWV>
+TL_DEV void qkv_rope_epilogue(const GemmArgs& a, const QkvRopeArgs& f, const QkvRopeOps<NE>& o, const int* red,
                               int lane) {
-    constexpr int NBLK = 4, NE = 8;
     const int d = lane & 31, D = f.n_heads * kHeadDim;
     int a0[NE], a1[NE];   // every partial sum first: the LDS reads overlap
 #pragma unroll
@@ -686,7 +687,7 @@ TL_DEV void qkv_rope_epilogue(const GemmArgs& a, const QkvRopeArgs& f, const Qkv
         a0[ee] = 0;
         a1[ee] = 0;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
+        for (int w = 0; w < NWV; w++) {
             a0[ee] += red[((w * NBLK + o.i * 2) * 16 + e) * 64 + lane];
             a1[ee] += red[((w * NBLK + o.i * 2 + 1) * 16 + e) * 64 + lane];
         }
@@ -733,12 +734,13 @@ struct SplitOps {
     float sw[NBW];
 };
 
-template <int TM, int TN, int EPI>
-__global__ __launch_bounds__(256) void gemm_pk_split_kernel(GemmArgs a, QkvRopeArgs f) {
+template <int TM, int TN, int EPI, int NWV = 4>
+__global__ __launch_bounds__(NWV * 64) void gemm_pk_split_kernel(GemmArgs a, QkvRopeArgs f) {
+    static_assert(NWV == 4 || EPI == EPI_QKV_ROPE, "the plain epilogue deals blocks to four wavefronts");
     constexpr int NF = TM + TN, PD = kPkSplitPD, NBLK = TM * TN, NBW = (NBLK + 3) / 4;
     constexpr bool RES = EPI == EPI_DEQUANT_RES;
-    extern __shared__ __align__(16) int pk_red[];   // [4 waves][NBLK][16][64]
-    const int kc = a.k >> 5, per = kc >> 2;        // chunks of each wavefront (a multiple of PD)
+    extern __shared__ __align__(16) int pk_red[];   // [NWV][NBLK][16][64]
+    const int kc = a.k >> 5, per = kc / NWV;        // chunks of each wavefront (a multiple of PD)
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const int mt0 = blockIdx.y * TM, nt0 = blockIdx.x * TN, c0 = wave * per;
     const int8_t* ab = a.ap + lane * 16;
@@ -787,10 +789,11 @@ __global__ __launch_bounds__(256) void gemm_pk_split_kernel(GemmArgs a, QkvRopeA
     // (vector-memory waits complete in issue order, so issued earlier they
     // would hold up the main loop's waits).  Block b, lane l, register e is
     // output row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32.
-    QkvRopeOps qo;
+    constexpr int NE = EPI == EPI_QKV_ROPE ? 16 * TM / NWV : 1;
+    QkvRopeOps<NE> qo;
     SplitOps<NBW, RES> so;
     if constexpr (EPI == EPI_QKV_ROPE) {
-        static_assert(TM == 2 && TN == 2, "one 64-row x one-head tile");
+        static_assert(TN == 2 && 16 * TM % NWV == 0, "one head, whole rows per wavefront");
         qkv_rope_operands(a, f, mt0, nt0, wave, lane, qo);
     } else {
 #pragma unroll
@@ -818,7 +821,7 @@ __global__ __launch_bounds__(256) void gemm_pk_split_kernel(GemmArgs a, QkvRopeA
     if constexpr (EPI == EPI_QKV_ROPE) qkv_rope_tables(f, lane, qo);
     __syncthreads();
     if constexpr (EPI == EPI_QKV_ROPE) {
-        qkv_rope_epilogue(a, f, qo, pk_red, lane);
+        qkv_rope_epilogue<NE, NBLK, NWV>(a, f, qo, pk_red, lane);
         return;
     }
     // wavefront w finishes blocks w, w + 4, ... (y may be the residual, read
@@ -1045,6 +1048,13 @@ hipError_t launch_gemm_pk_qkv(hipStream_t s, const GemmArgs& a, const QkvRopeArg
     if (!a.ap || !a.wp || !f.q_out || !f.q_max || f.n_heads <= 0 || f.n_kv <= 0 || a.n != D + 2 * KVD ||
         a.k % 512 || a.n % 64)
         return hipErrorInvalidValue;
+    if (a.m <= 32 && a.k % 1024 == 0) {
+        // one row block: 8 wavefronts split K, 32 x 64 tiles (latency bound: 40
+        // workgroups of 4 wavefronts and 64-row tiles took 9.2 us at 20 rows, this 5.5)
+        TL_KLAUNCH((gemm_pk_split_kernel<1, 2, EPI_QKV_ROPE, 8>), dim3(a.n / 64, 1), dim3(512),
+                   pk_split_lds_bytes(1, 2, 8), s, a, f);
+        return hipGetLastError();
+    }
     TL_KLAUNCH((gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>), dim3(a.n / 64, (a.m + 63) / 64), dim3(256),
                pk_split_lds_bytes(2, 2), s, a, f);
     return hipGetLastError();
@@ -1055,10 +1065,12 @@ hipError_t init_gemm_pk_kernels() {
                          (const void*)gemm_pk_split_kernel<1, 5, EPI_DEQUANT_RES>,
                          (const void*)gemm_pk_split_kernel<2, 2, EPI_DEQUANT>,
                          (const void*)gemm_pk_split_kernel<2, 2, EPI_DEQUANT_RES>, (const void*)gemm_pk_glu_kernel<1>,
-                         (const void*)gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>};
+                         (const void*)gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>,
+                         (const void*)gemm_pk_split_kernel<1, 2, EPI_QKV_ROPE, 8>};
     const size_t bytes[] = {pk_split_lds_bytes(1, 5), pk_split_lds_bytes(1, 5), pk_split_lds_bytes(2, 2),
-                            pk_split_lds_bytes(2, 2), pk_glu_lds_bytes(1), pk_split_lds_bytes(2, 2)};
-    for (int i = 0; i < 6; i++) {
+                            pk_split_lds_bytes(2, 2), pk_glu_lds_bytes(1), pk_split_lds_bytes(2, 2),
+                            pk_split_lds_bytes(1, 2, 8)};
+    for (int i = 0; i < 7; i++) {
         const hipError_t e = hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes[i]);
         if (e != hipSuccess) return e;
     }
