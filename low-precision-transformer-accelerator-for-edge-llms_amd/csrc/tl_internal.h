@@ -206,11 +206,12 @@ constexpr int kTileMaxKeys = 4096;   // context limit of launch_attention_tiles 
 // qf / qmax (optional, instead of q8 / q_scale): rotated Q rows in float32
 // ([rows][D]) and their maxima max|q| as float bits ([rows][kQmaxStride],
 // element 0),
-// quantized by the kernel exactly as qkv_post quantizes them
+// quantized by the kernel exactly as qkv_post quantizes them; out_max (optional):
+// [rows][n_heads] max |output| of each head
 hipError_t launch_attention_tiles(hipStream_t s, const int8_t* q8, const double* q_scale, int32_t rows,
                                   int32_t n_heads, int32_t n_kv_heads, int32_t seq, int32_t pos0, KvGeom kv,
                                   int32_t layer, const float* kv_sk, const float* kv_sv, float* out,
-                                  const float* qf = nullptr, const unsigned* qmax = nullptr);
+                                  const float* qf = nullptr, const unsigned* qmax = nullptr, float* out_max = nullptr);
 // Optional debug outputs of row 0 (the decode-step capture): INT32 scores and
 // INT8 probabilities of keys key0 .. key0 + n_keys - 1 per query head
 // ([n_heads][n_keys]) and the f32 score scale per query head.

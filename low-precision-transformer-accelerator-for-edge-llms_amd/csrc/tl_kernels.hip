@@ -960,6 +960,7 @@ struct AttnTileArgs {
     float* out;              // [rows][D]
     const float* qf;         // or rotated Q in float32 [rows][D], quantized here
     const unsigned* qmax;    // with qf: max|q| of each row as float bits [rows][kQmaxStride]
+    float* out_max;          // or null: [rows][n_heads] max |out| of each head
 };
 
 // Q fragments of a tile lane (row r, head h, K halves hi * 16 .. + 16 and
@@ -1213,9 +1214,15 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_kernel(AttnTileArgs
     }
     __syncthreads();
     const float pv_mult = deq_mult(1.0 / 127.0, sv);
-    for (int e = tid; e < 32 * 64; e += NW * 64) {
+    for (int e = tid; e < 32 * 64; e += NW * 64) {   // one row per wavefront
         const int r = e >> 6, d = e & 63;
-        if (r < nr) p.out[(int64_t)(r0 + r) * D + (int64_t)h * kHeadDim + d] = (float)accs[e] * pv_mult;
+        if (r >= nr) break;
+        const float v = (float)accs[e] * pv_mult;
+        p.out[(int64_t)(r0 + r) * D + (int64_t)h * kHeadDim + d] = v;
+        if (p.out_max) {   // the head's part of the maximum the O projection quantizes the row at
+            const float mx = wave_max_f32(fabsf(v));
+            if (d == 0) p.out_max[(int64_t)(r0 + r) * p.n_heads + h] = mx;
+        }
     }
 }
 
@@ -2275,9 +2282,15 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_reg_kernel(AttnTile
     }
     __syncthreads();
     const float pv_mult = deq_mult(1.0 / 127.0, sv);
-    for (int e = tid; e < 32 * 64; e += NW * 64) {
+    for (int e = tid; e < 32 * 64; e += NW * 64) {   // one row per wavefront
         const int r = e >> 6, d = e & 63;
-        if (r < nr) p.out[(int64_t)(r0 + r) * D + (int64_t)h * kHeadDim + d] = (float)accs[e] * pv_mult;
+        if (r >= nr) break;
+        const float v = (float)accs[e] * pv_mult;
+        p.out[(int64_t)(r0 + r) * D + (int64_t)h * kHeadDim + d] = v;
+        if (p.out_max) {   // the head's part of the maximum the O projection quantizes the row at
+            const float mx = wave_max_f32(fabsf(v));
+            if (d == 0) p.out_max[(int64_t)(r0 + r) * p.n_heads + h] = mx;
+        }
     }
 }
 
@@ -2285,14 +2298,14 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_reg_kernel(AttnTile
 hipError_t launch_attention_tiles(hipStream_t s, const int8_t* q8, const double* q_scale, int32_t rows,
                                   int32_t n_heads, int32_t n_kv_heads, int32_t seq, int32_t pos0, KvGeom kv,
                                   int32_t layer, const float* kv_sk, const float* kv_sv, float* out,
-                                  const float* qf, const unsigned* qmax) {
+                                  const float* qf, const unsigned* qmax, float* out_max) {
     if (rows <= 0) return hipSuccess;
     if (n_heads % n_kv_heads || pos0 < 0 || pos0 + rows > kv.max_pos || pos0 + rows > kTileMaxKeys ||
         (qf && !qmax) || (!qf && (!q8 || !q_scale)))
         return hipErrorInvalidValue;
     const int tpad = (pos0 + rows + 63) & ~63;
     AttnTileArgs a{q8, q_scale, n_heads, n_kv_heads, rows, seq, pos0, layer, kv, kv_sk, kv_sv,
-                   1.0 / sqrt((double)kHeadDim), out, qf, qmax};
+                   1.0 / sqrt((double)kHeadDim), out, qf, qmax, out_max};
     const dim3 grid(n_heads, (rows + 31) / 32), block(256);
     // Wavefronts per tile: one 64-key block each while the context allows
     // (up to 512 keys; up to 1024 while one round of 16-wavefront workgroups

@@ -704,22 +704,23 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
     // up to 32 rows of a batch or a prompt: the row kernels prefetch the next
     // GEMM's weight tiles, with a row kernel to fold it the down GEMM is
     // K-sliced, and a prompt's Q|K|V GEMM does qkv_post's work (fq), one launch
-    // less: one layer over 5 rows 88 -> 77 us, 32 rows 104 -> 87 us, 22 layers and the
-    // head over 20 rows 1.38 -> 1.26 ms, 32 rows 1.54 -> 1.30 ms (K slices
-    // and the head on packed weights give most of the latter two)
+    // less: one layer over 5 rows 88 -> 77 us, 32 rows 104 -> 87 us, a prompt of 20
+    // tokens with logits 1.38 -> 1.26 ms, of 32 1.54 -> 1.30 ms
     const bool few = kslice_ok(h, L, rows);
     const bool ks = few && chain;
     const bool qks = ks && decode && qkv_kslice_ok(h, L, rows, max_t);
-    // the O GEMM K-sliced with the attention output quantized in it (one
-    // 32-byte K chunk per wavefront of the 16-wavefront small-M GEMM)
-    const bool of = qks && h->o_fuse && L.wo_p && c.n_heads <= 32 && c.n_heads % 4 == 0 &&
-                    kslice_len(D, D) / 32 <= 16;
     const bool pk = (!decode || rows > 32) && prefill_packed(h, L, rows);   // h->a8 in the packed GEMM operand layout
     // prefill tiles on packed operands: qkv_post's work in the Q|K|V GEMM
     // epilogue, rotated Q in h->qkv ([rows][D]) quantized by the attention tiles
     // (up to 32 rows only the operand of that GEMM is packed)
     const bool fq = (pk || (few && !decode && L.wqkv_p && gemm_pk_supported(EPI_DEQUANT, rows, QKV, D))) &&
                     h->rows_one_seq && h->rows_pos0 + rows <= kTileMaxKeys && D % 64 == 0 && KVD % 64 == 0;
+    // up to 32 rows: the O GEMM K-sliced with the attention output quantized in it
+    // (one 32-byte K chunk per wavefront of the 16-wavefront small-M GEMM); for a
+    // prompt one launch of nine less: with logits, 3 tokens 1.11 -> 1.03 ms, 20
+    // 1.21 -> 1.15, 32 1.27 -> 1.20 ms
+    const bool of = (qks || (few && fq)) && h->o_fuse && L.wo_p && c.n_heads <= 32 && c.n_heads % 4 == 0 &&
+                    kslice_len(D, D) / 32 <= 16;
     // The row kernel before a GEMM also brings that GEMM's packed weight tiles
     // into the L2 of the XCD whose workgroups read them: the packed GEMMs'
     // grids have a multiple of 8 column tiles in x, so column tile t runs on
@@ -769,7 +770,8 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
     } else if (fq) {
         Prof p(h, TL_K_ATTN, (double)rows * c.n_kv_heads * (double)max_t * 128.0 + rows * D * 8.0);
         TL_LAUNCH(h, launch_attention_tiles(h->stream, nullptr, nullptr, rows, c.n_heads, c.n_kv_heads, h->rows_seq,
-                                            h->rows_pos0, h->kv, layer, h->kv_sk, h->kv_sv, h->att, h->qkv, h->qmax));
+                                            h->rows_pos0, h->kv, layer, h->kv_sk, h->kv_sv, h->att, h->qkv, h->qmax,
+                                            of ? h->att_max : nullptr));
     } else {
         {
             Prof p(h, TL_K_ATTN, (double)rows * (QKV * 4.0 + D) + (double)rows * KVD * 2.0);
@@ -783,7 +785,8 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
         // the O GEMM K-sliced over the chip, quantizing the float32 attention
         // output itself at each row's maximum (from the heads' maxima); its
         // integer sums wait in h->racc for the post-attention RMSNorm, which
-        // adds them to the residual and also clears the Q|K|V sums
+        // adds them to the residual and also clears the Q|K|V sums (or the Q row
+        // maxima)
         GemmArgs a{};
         a.a = h->a8; a.af = h->att; a.amax = h->att_max; a.amax_n = c.n_heads; a.as_out = h->as;
         a.wp = L.wo_p; a.acc = h->racc; a.m = rows; a.n = D; a.k = D; a.k_split = kslice_len(D, D);
@@ -795,14 +798,14 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
         FoldArgs f{};
         f.x = h->x; f.acc = h->racc; f.as = h->as; f.ws = L.so; f.g = L.g_post;
         f.rows = rows; f.n = D; f.eps = c.rms_eps; f.plan = h->plan; f.q = h->a8; f.scales = h->as;
-        f.zero = h->qacc; f.zero_n = QKV;
+        f.zero = qks ? h->qacc : (int32_t*)h->qmax; f.zero_n = qks ? QKV : kQmaxStride;
         if (l2pf) f.pf = pf_glu;
         {
-            Prof p(h, TL_K_NORM, (double)rows * D * 13.0 + (double)rows * QKV * 4.0);
+            Prof p(h, TL_K_NORM, (double)rows * D * 13.0 + (double)rows * f.zero_n * 4.0);
             TL_LAUNCH(h, launch_rows_fold(h->stream, f));
         }
         h->racc_clean = true;
-        h->qacc_clean = true;
+        (qks ? h->qacc_clean : h->qmax_clean) = true;
     } else {
         {
             // with the Q|K|V sums (or the Q row maxima) consumed, this kernel also
