@@ -1048,15 +1048,18 @@ hipError_t launch_gemm_pk_qkv(hipStream_t s, const GemmArgs& a, const QkvRopeArg
     if (!a.ap || !a.wp || !f.q_out || !f.q_max || f.n_heads <= 0 || f.n_kv <= 0 || a.n != D + 2 * KVD ||
         a.k % 512 || a.n % 64)
         return hipErrorInvalidValue;
-    if (a.m <= 32 && a.k % 1024 == 0) {
-        // one row block: 8 wavefronts split K, 32 x 64 tiles (latency bound: 40
-        // workgroups of 4 wavefronts and 64-row tiles took 9.2 us at 20 rows, this 5.5)
-        TL_KLAUNCH((gemm_pk_split_kernel<1, 2, EPI_QKV_ROPE, 8>), dim3(a.n / 64, 1), dim3(512),
+    const int rt = (a.m + 31) / 32;
+    if ((a.n / 64) * rt <= 512 && a.k % 1024 == 0) {
+        // 32 x 64 tiles, 8 wavefronts split K (latency bound; against 64 x 64
+        // tiles of 4 wavefronts at 20, 45, 100, 190 rows 5.5, 5.5, 6.0, 6.6 us for 9.2, 8.6,
+        // 9.0, 9.6) while all tiles are resident, two per CU (256 rows 9.3 for 10.0,
+        // 384 rows 10.4 for 10.4); 64 x 64 of 8 wavefronts 7.9-8.8 us to 256 rows
+        TL_KLAUNCH((gemm_pk_split_kernel<1, 2, EPI_QKV_ROPE, 8>), dim3(a.n / 64, rt), dim3(512),
                    pk_split_lds_bytes(1, 2, 8), s, a, f);
         return hipGetLastError();
     }
-    TL_KLAUNCH((gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>), dim3(a.n / 64, (a.m + 63) / 64), dim3(256),
-               pk_split_lds_bytes(2, 2), s, a, f);
+    const dim3 grid(a.n / 64, (a.m + 63) / 64);
+    TL_KLAUNCH((gemm_pk_split_kernel<2, 2, EPI_QKV_ROPE>), grid, dim3(256), pk_split_lds_bytes(2, 2), s, a, f);
     return hipGetLastError();
 }
 

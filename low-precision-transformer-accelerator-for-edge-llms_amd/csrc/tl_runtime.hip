@@ -119,7 +119,7 @@ struct tl_handle {
     float* rope_cos = nullptr;
     float* rope_sin = nullptr;
     int32_t rope_n = 0;
-    float* att_max = nullptr;   // [max rows][n_heads]: each head's max |attention output| (batched decode)
+    float* att_max = nullptr;   // [max rows][n_heads]: each head's max |attention output| (up to 32 rows)
     int32_t* pf_sink = nullptr; // written by the L2 prefetch workgroups only if their loads XOR to a magic value
     float* kv_sk = nullptr;
     float* kv_sv = nullptr;
@@ -145,7 +145,7 @@ struct tl_handle {
     unsigned long long* op_key = nullptr;  // argmax slot of the standalone LM-head operator
     unsigned long long* lm_wg_keys = nullptr;  // [vocab / 4] batch-1 LM head: argmax key per workgroup
     int32_t* partials = nullptr;
-    int32_t* racc = nullptr;      // [32][D] integer sums of the K-sliced batched-decode down GEMM; zero
+    int32_t* racc = nullptr;      // [32][D] integer sums of the K-sliced O and down GEMMs of up to 32 rows; zero
                                   // between uses (the fold prologue clears what it read)
     size_t racc_cap = 0;          // int32 elements
     int32_t* qacc = nullptr;      // [32][QKV] integer sums of the K-sliced batched-decode Q|K|V GEMM, read
@@ -184,7 +184,7 @@ struct tl_handle {
     std::string err;
 
 
-    bool batch_kslice = true;             // batched decode: K-sliced down GEMM folded by the next RMSNorm
+    bool batch_kslice = true;             // up to 32 rows: K-sliced down GEMM folded by the next RMSNorm
                                           // row prologue (TL_BATCH_KSLICE=0 turns it off)
     const float* racc_res_ws = nullptr;   // racc holds a down projection's sums (these weight scales) that
                                           // the next RMSNorm prologue adds to h->x
@@ -192,7 +192,7 @@ struct tl_handle {
     bool qkv_kslice = true;               // batched decode: K-sliced Q|K|V GEMM whose sums the attention
                                           // kernel dequantizes (TL_BATCH_QKV_KSLICE=0 turns it off)
     bool qacc_clean = true;               // false from a Q|K|V EPI_ACC launch until qacc is cleared
-    bool o_fuse = true;                   // batched decode: the O GEMM K-sliced, quantizing the attention output itself
+    bool o_fuse = true;                   // up to 32 rows: the O GEMM K-sliced, quantizing the attention output itself
                                           // at the row maxima the attention kernel leaves; its sums folded by the
                                           // post-attention RMSNorm (TL_BATCH_O_FUSE=0 turns it off)
     bool qmax_clean = true;               // false from a fused Q|K|V GEMM until qmax is cleared

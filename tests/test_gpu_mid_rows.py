@@ -136,12 +136,15 @@ def test_decode_crosses_a_context_bound(n, new):
     eng.close()
 
 
-@pytest.mark.parametrize("n", [2, 5, 31, 32, 33])
-def test_short_prompt_chains_layers(n):
+@pytest.mark.parametrize("n,off", [(2, None), (5, None), (31, None), (32, None), (33, None), (20, "TL_BATCH_O_FUSE"),
+                                   (20, "TL_BATCH_KSLICE")])
+def test_short_prompt_chains_layers(monkeypatch, n, off):
     """Prompts of up to 32 rows leave each layer's down projection as integer sums that the next layer's RMSNorm
-    folds, and the last layer's complete: the logits of every position, the caches of all layers and a single-layer
+    folds, and the last layer's complete (and the forms with these fusions switched off): the logits of every position, the caches of all layers and a single-layer
     call after the prompt equal the oracle's."""
     from lpta.engine import Engine
+    if off:
+        monkeypatch.setenv(off, "0")
     cfg = dict(oracle.TINYLLAMA_CFG, n_layers=3, vocab=512)
     m = oracle.synthetic_model(cfg, seed=500 + n)
     eng = Engine(m.cfg, max_seqs=1).load_model(m)
