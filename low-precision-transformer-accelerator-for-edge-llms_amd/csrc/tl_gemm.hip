@@ -613,9 +613,9 @@ TL_DEV void pk_wait_regs(v4i* r) {
 // and wavefront w finishes blocks w, w + 4, ... of the tile with the epilogue
 // arithmetic of every other GEMM here.  Tiles: 64 x 64 (TM = TN = 2) for O and
 // down (256 workgroups at M = 512), 32 x 160 (TM = 1, TN = 5) for Q|K|V
-// (N = 2560: 256 workgroups where 64 x 64 needs 320); 64 x 64 for the
-// prefill Q|K|V with qkv_post's work in the epilogue (EPI_QKV_ROPE, one head
-// per tile).  The epilogue's operands are loaded behind the last operand
+// (N = 2560: 256 workgroups where 64 x 64 needs 320); for the prefill Q|K|V
+// with qkv_post's work in the epilogue (EPI_QKV_ROPE, one head per tile) 32 x 64
+// with 8 wavefronts over eighths of K, or 64 x 64 (launch_gemm_pk_qkv).  The epilogue's operands are loaded behind the last operand
 // loads, so they arrive during the last MFMAs.
 constexpr int kPkSplitPD = 4;
 

@@ -425,7 +425,7 @@ int32_t run_gemm(tl_handle* h, int epi, GemmArgs a, int kclass, const FixedScrat
     }
     if (a.m <= 32 && a.wp && (epi != EPI_GLU || (a.wp2 && a.k <= 2048)) && a.k % 64 == 0 && a.k <= 6144 &&
         a.n % 32 == 0) {
-        // batched decode on the packed weight copies: one 16-wavefront
+        // batched decode and short prompts on the packed weight copies: one 16-wavefront
         // workgroup per 32 output columns, every weight load a coalesced 1 KiB
         // (measured faster than splitting K over workgroups: the cross-XCD
         // reduction of the partial tiles costs more than the added bandwidth)
@@ -725,8 +725,8 @@ int32_t layer_rows(tl_handle* h, int32_t layer, int32_t rows, int32_t max_t, boo
     // into the L2 of the XCD whose workgroups read them: the packed GEMMs'
     // grids have a multiple of 8 column tiles in x, so column tile t runs on
     // XCD t % 8 (batched decode: 32-column tiles; prefill: 64-column tiles,
-    // gate/up's 32).  Batched decode prefetches for Q|K|V, gate/up and down
-    // (O follows attention, not a row kernel); prefill for all four.
+    // gate/up's 32).  Up to 32 rows prefetch for Q|K|V, gate/up and down (O
+    // follows attention, not a row kernel); longer prompts for all four.
     auto pf_plan = [&](const int8_t* w0, const int8_t* w1, int nmat, int cols, int n, int k) {
         L2Prefetch p{};
         p.w[0] = w0;
