@@ -144,7 +144,8 @@ struct tl_handle {
     float* fscratch = nullptr;    // small scratch
     unsigned long long* op_key = nullptr;  // argmax slot of the standalone LM-head operator
     unsigned long long* lm_wg_keys = nullptr;  // [vocab / 4] batch-1 LM head: argmax key per workgroup
-    int32_t* partials = nullptr;
+    unsigned long long* tile_keys = nullptr;   // [vocab / 32][max_seqs] LM head of many rows: best key of 32 columns
+    int32_t* partials = nullptr;  // split-K scratch, grown on demand (ensure_partials)
     int32_t* racc = nullptr;      // [32][D] integer sums of the K-sliced O and down GEMMs of up to 32 rows; zero
                                   // between uses (the fold prologue clears what it read)
     size_t racc_cap = 0;          // int32 elements
@@ -363,12 +364,24 @@ int32_t finish(tl_handle* h) {
 }
 
 // ---- GEMM dispatch: M == 1 uses the GEMV kernels, M > 1 the MFMA kernels ----
+
+// h->partials of at least `need` elements.  A captured batch step may hold the
+// buffer's address (split-K GEMMs of batches that the packed tiles do not take),
+// so all of them are dropped when the buffer moves and captured again on their
+// next use.  Never grows inside a capture: a call's first step runs eagerly
+// with the same GEMMs (and the wait below refuses a capturing stream).
 int32_t ensure_partials(tl_handle* h, size_t need) {
     if (need <= h->partial_cap) return TL_OK;
     if (h->partials) {
+        TL_HIP(h, hipStreamSynchronize(h->stream));
+        for (hipGraphExec_t& g : h->batch_graphs) {
+            if (g) (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
         (void)hipFree(h->partials);
         h->allocs.erase(std::remove(h->allocs.begin(), h->allocs.end(), (void*)h->partials), h->allocs.end());
         h->partials = nullptr;
+        h->partial_cap = 0;
     }
     TL_HIP(h, dalloc(h, &h->partials, need));
     h->partial_cap = need;
@@ -884,10 +897,8 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
             // MFMA GEMM (up to 32 rows on the packed weights) with the argmax in its
             // epilogue, one key per 32 columns and row, then these keys folded per row
             const int tiles = V / 32;
-            int32_t r = ensure_partials(h, (size_t)tiles * rows * 2);
-            if (r) return r;
             a.wp = h->lm_wp;
-            a.key = (unsigned long long*)h->partials;
+            a.key = h->tile_keys;
             a.y = nullptr;
             Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + (double)rows * D);
             if (lm_tile) TL_LAUNCH(h, launch_gemm32(h->stream, EPI_ARGMAX, a, true));
@@ -1036,8 +1047,9 @@ int32_t decode_graph_launch(tl_handle* h, int32_t seq, int32_t max_t) {
 // one batched decode step of sequences 0..n_seqs-1 (rows r = sequence r):
 // embed each sequence's current token at its cursor, the decoder layers at
 // M = n_seqs, the LM head with its argmax, then record the tokens and advance
-// the cursors.  Every argument is a fixed device pointer, so the step can be
-// captured once per batch size and replayed.
+// the cursors.  Every argument is a fixed device pointer (h->partials until it
+// grows, which drops the captured steps), so the step can be captured once per
+// batch size and replayed.
 int32_t batch_step(tl_handle* h, int32_t n_seqs, int32_t max_t) {
     const tl_config& c = h->cfg;
     int32_t r;
@@ -1149,6 +1161,7 @@ int32_t tl_create(const tl_config* cfg, int32_t max_seqs, tl_handle** out) {
         (e = dalloc(h, &h->row_pos, (size_t)R)) || (e = dalloc(h, &h->tokens, (size_t)R)) ||
         (e = dalloc(h, &h->fscratch, 64)) || (e = dalloc(h, &h->op_key, 1)) || (e = dalloc(h, &h->keys, (size_t)max_seqs)) ||
         (e = dalloc(h, &h->lm_wg_keys, (size_t)(c.vocab + 3) / 4)) ||
+        (e = dalloc(h, &h->tile_keys, (size_t)(c.vocab / 32) * max_seqs)) ||
         (e = dalloc(h, &h->token_cur, (size_t)max_seqs)) || (e = dalloc(h, &h->cursor, (size_t)max_seqs)) ||
         (e = dalloc(h, &h->n_gen, (size_t)max_seqs)) || (e = dalloc(h, &h->eos_id, (size_t)max_seqs)) ||
         (e = dalloc(h, &h->stopped, (size_t)max_seqs)) ||
@@ -1937,8 +1950,8 @@ int32_t tl_decode_batch(tl_handle* h, int32_t n_seqs, const int32_t* tokens, con
     TL_HIP(h, hipMemcpyAsync(h->cursor, start_pos, sizeof(int32_t) * n_seqs, hipMemcpyHostToDevice, h->stream));
     TL_HIP(h, hipMemcpyAsync(h->n_gen, zeros.data(), sizeof(int32_t) * n_seqs, hipMemcpyHostToDevice, h->stream));
     TL_LAUNCH(h, launch_reset_keys(h->stream, h->keys, n_seqs));
-    // the first step runs eagerly (it sizes the scratch the LM head's tile
-    // keys need), the rest replay the captured step
+    // the first step runs eagerly (it sizes the scratch split-K GEMMs need),
+    // the rest replay the captured step
     for (int step = 0; step < n_steps; step++) {
         if (step > 0 && !h->profiling) {
             if ((r = batch_graph_launch(h, n_seqs, max_t))) return r;

@@ -66,6 +66,39 @@ def test_decode_batch_rows_and_context_bounds(B, top):
     eng.close()
 
 
+def test_decode_batch_sizes_alternate_on_one_engine():
+    """Captured batch steps stay valid when the split-K scratch moves: on one
+    engine, batches of 4, 40 (split-K projections: this intermediate width has no packed
+    form), 60 and a scored prompt of 63 tokens, each needing more scratch than
+    the one before, and then 4 and 40 again give the oracle's ids."""
+    from lpta.engine import Engine
+    cfg = dict(oracle.SMALL_CFG)
+    m = oracle.synthetic_model(cfg, seed=91)
+    eng = Engine(m.cfg, max_seqs=60).load_model(m)
+    orc = oracle.Oracle(m)
+    rng = np.random.default_rng(91)
+    toks = rng.integers(0, cfg["vocab"], 60).astype(np.int32)
+    steps = 4   # an eager one and three replays
+    caches = [m.new_cache() for _ in range(60)]
+    want, tok = [], toks
+    for p in range(steps):   # sequences of a batch are independent: the first B of 60
+        x = np.stack([orc.embed(int(t)) for t in tok]).astype(F32)
+        for layer in range(cfg["n_layers"]):
+            orc.decode_rows(layer, np.full(60, p, np.int32), x, caches)
+        tok, _ = orc.lm_head_rows(x)
+        tok = np.asarray(tok, np.int32)
+        want.append(tok)
+    want = np.stack(want, 1)
+    logits = dev(np.zeros((63, cfg["vocab"]), F32))
+    for b in (4, 40, 60, None, 4, 40, 60):
+        if b is None:
+            eng.rt.call("tl_prefill_logits", 0, rng.integers(0, cfg["vocab"], 63).astype(np.int32), 63, logits)
+            continue
+        got = eng.decode_batch(toks[:b], np.zeros(b, np.int32), steps)
+        assert_bits_equal(np.asarray(got, np.int32), want[:b], f"batch of {b}")
+    eng.close()
+
+
 @pytest.fixture(scope="module")
 def layer_eng():
     from lpta.engine import Engine
