@@ -25,38 +25,39 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 // What bounds it: the float32 matrix rate at hundreds of rows (640 x 5632 x
 // 2048: 90 TFLOP/s; 100 x 5632 x 2048 puts 236 of 256 CUs at work), launch and
 // latency at a few.  The whole call at 100 x 5632 x 2048: 245 us with 64 x 64 vector-FMA
-// tiles through LDS, 53 us now; 640 rows 407 -> 175; one row 238 -> 30.  Eight
+// tiles through LDS, 51 us now; 640 rows 407 -> 167; one row 238 -> 28.  Eight
 // partial sums per output also round less: 2.9e-7 relative to 64 bits where
 // one chain of 2048 had 8.1e-7.
 constexpr int kLinWaves = 8;
 
-template <int NB, bool VEC>
+// OFF: unsigned lane offsets of elements, or int64_t where 32 k or 8 n passes 2^32
+template <int NB, bool VEC, typename OFF>
 __global__ __launch_bounds__(kLinWaves * 64) void linear_f32_kernel(const float* __restrict__ x,
                                                                     const float* __restrict__ w,
                                                                     const float* __restrict__ b,
                                                                     const float* __restrict__ residual, int32_t m,
-                                                                    int32_t n, int32_t k, int32_t tiles_m,
-                                                                    int32_t tiles_n, float* __restrict__ y) {
+                                                                    int32_t n, int32_t k, int32_t tiles_n,
+                                                                    float* __restrict__ y) {
     constexpr int PD = NB == 1 ? 8 : 4, HW = kLinWaves / 2;   // chunks in flight; LDS partial tiles
     __shared__ float red[HW][NB * 16][64];
-    // workgroups go to the 8 XCDs round-robin: the row tiles of a column tile
-    // stay on one XCD, whose L2 then holds the column tile's weights
-    const int q = (int)blockIdx.x >> 3, tn = q / tiles_m * 8 + ((int)blockIdx.x & 7), tm = q % tiles_m;
+    // workgroups go to the 8 XCDs round-robin in x (8 x the row tiles), y, z order: the
+    // row tiles of a column tile stay on one XCD, whose L2 then holds the column
+    // tile's weights
+    const int tm = (int)blockIdx.x >> 3, tn = (int)(blockIdx.z * gridDim.y + blockIdx.y) * 8 + ((int)blockIdx.x & 7);
     if (tn >= tiles_n) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), col = lane & 31, hi = lane >> 5;
     const int64_t row0 = (int64_t)tm * 32;
-    const int col0 = tn * 32 * NB;
-    const int nfull = k >> 3, nch = (k + 7) >> 3, per = (nch + kLinWaves - 1) / kLinWaves;
+    const unsigned col0 = (unsigned)tn * 32 * NB;   // column indices pass 2^31 in the last tile of the widest n
+    const int nfull = k >> 3, nch = nfull + ((k & 7) != 0), per = (nch + kLinWaves - 1) / kLinWaves;
     const int c0 = min(wave * per, nfull), c1 = min(c0 + per, nfull);   // this wavefront's whole chunks
-    // one wavefront-uniform base per chunk and 32-bit lane offsets: no 64-bit
-    // address arithmetic per load
+    // one wavefront-uniform base per chunk, and lane offsets formed once
     const float* xb = x + row0 * k;
-    const unsigned xo = (unsigned)min(col, (int)(m - 1 - row0)) * (unsigned)k + 4 * hi;
-    unsigned wo[4][NB];
+    const OFF xo = (OFF)min(col, (int)(m - 1 - row0)) * (OFF)k + 4 * hi;
+    OFF wo[4][NB];
 #pragma unroll
     for (int s = 0; s < 4; s++)
 #pragma unroll
-        for (int j = 0; j < NB; j++) wo[s][j] = (unsigned)(4 * hi + s) * (unsigned)n + (unsigned)min(col0 + 32 * j + col, n - 1);
+        for (int j = 0; j < NB; j++) wo[s][j] = (OFF)(4 * hi + s) * (OFF)n + min(col0 + 32 * j + col, (unsigned)n - 1);
     v16f acc[NB];
 #pragma unroll
     for (int j = 0; j < NB; j++) acc[j] = (v16f){};
@@ -130,8 +131,8 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_f32_kernel(const float*
     for (int i = 0; i < 2 * NB; i++) {   // output register e of block j: 16 NB of them over 8 wavefronts
         const int je = i * kLinWaves + wave, e = je & 15;
         const int64_t r = row0 + 8 * (e >> 2) + 4 * hi + (e & 3);
-        const int c = col0 + 32 * (je >> 4) + col;
-        if (r >= m || c >= n) continue;
+        const unsigned c = col0 + 32 * (je >> 4) + col;
+        if (r >= m || c >= (unsigned)n) continue;
         float v = (red[0][je][lane] + red[1][je][lane]) + (red[2][je][lane] + red[3][je][lane]);
         if (b) v = v + b[c];
         const int64_t idx = r * n + c;
@@ -140,14 +141,23 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_f32_kernel(const float*
     }
 }
 
+template <int NB, bool VEC, typename OFF>
+void go_linear_kernel(hipStream_t s, const float* x, const float* w, const float* b, const float* residual, int32_t m,
+                      int32_t n, int32_t k, float* y) {
+    // three grid dimensions: one would pass the limit of 2^32 threads at 8.4 million tiles
+    constexpr int32_t kMaxY = 32768;
+    const int32_t tm = (int32_t)(((int64_t)m + 31) / 32), tn = (int32_t)(((int64_t)n + 32 * NB - 1) / (32 * NB));
+    const int32_t cols8 = (tn + 7) / 8;   // groups of 8 column tiles, one per XCD
+    const dim3 grid(8u * (unsigned)tm, std::min(cols8, kMaxY), (cols8 + kMaxY - 1) / kMaxY);
+    TL_KLAUNCH((linear_f32_kernel<NB, VEC, OFF>), grid, dim3(kLinWaves * 64), 0, s, x, w, b, residual, m, n, k, tn, y);
+}
+
 template <int NB>
 void go_linear(hipStream_t s, const float* x, const float* w, const float* b, const float* residual, int32_t m,
                int32_t n, int32_t k, float* y) {
-    const int32_t tm = (int32_t)(((int64_t)m + 31) / 32), tn = (n + 32 * NB - 1) / (32 * NB);
-    const dim3 grid((unsigned)((tn + 7) / 8 * 8) * (unsigned)tm), block(kLinWaves * 64);
     if (k % 4 == 0 && (uintptr_t)x % 16 == 0)
-        TL_KLAUNCH((linear_f32_kernel<NB, true>), grid, block, 0, s, x, w, b, residual, m, n, k, tm, tn, y);
-    else TL_KLAUNCH((linear_f32_kernel<NB, false>), grid, block, 0, s, x, w, b, residual, m, n, k, tm, tn, y);
+        go_linear_kernel<NB, true, unsigned>(s, x, w, b, residual, m, n, k, y);
+    else go_linear_kernel<NB, false, unsigned>(s, x, w, b, residual, m, n, k, y);
 }
 
 // one (query row i, query head h) per workgroup; the row's scores live in LDS
@@ -222,6 +232,10 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
 hipError_t launch_linear_f32(hipStream_t s, const float* x, const float* w, const float* b, const float* residual,
                              int32_t m, int32_t n, int32_t k, float* y) {
     if (m <= 0 || n <= 0) return hipSuccess;
+    if (k >= 1 << 27 || n > 1 << 29) {   // lane offsets past 2^32
+        go_linear_kernel<1, false, int64_t>(s, x, w, b, residual, m, n, k, y);
+        return hipGetLastError();
+    }
     // column blocks per tile: the fewest MFMAs on the busiest CU (rounds of 256
     // tiles times blocks); of equals the widest, which reads x least often
     const int64_t tm = ((int64_t)m + 31) / 32;

@@ -63,3 +63,32 @@ def test_linear_f32_special_values(rt):
     assert (got[2] == F32(F64(x[2, 12]) * F64(w[12, 0]))).all()
     assert got[1, 7] == np.inf and np.isnan(got[1, 8])   # inf * 0
     assert got[3, 9] == np.inf and got[3, 8] == 0.0
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (32, 1, 138_547_336),    # 31 k = 2^32 + 120: the last row's offset from its tile
+    (2, 613_566_760, 8),     # 7 n = 2^32 + 24: the last row of W; 4.8 million column tiles
+])
+def test_linear_f32_offsets_past_32_bits(rt, m, n, k):
+    """Offsets inside a tile that pass 2^32 elements: all-zero operands with a
+    few small whole numbers in the first and last rows, columns and k's, whose
+    products no other place may show."""
+    import torch
+    x = torch.zeros((m, k), device="cuda")
+    w = torch.zeros((k, n), device="cuda")
+    ks = [0, 3, k // 2, k - 2, k - 1]   # distinct from k = 8
+    cols = sorted({0, n // 3, n - 1})
+    for i, kk in enumerate(ks):
+        for r in {0, m - 1}:
+            x[r, kk] = 1 + i + 7 * (r > 0)
+        for j, c in enumerate(cols):
+            w[kk, c] = 2 + 3 * i + 11 * j
+    y = torch.full((m, n), 9.0, device="cuda")
+    torch.cuda.synchronize()
+    rt.call("tl_linear_f32", x, w, None, None, m, n, k, y)
+    for r in {0, m - 1}:
+        for j, c in enumerate(cols):
+            want = sum((1 + i + 7 * (r > 0)) * (2 + 3 * i + 11 * j) for i in range(len(ks)))
+            assert float(y[r, c]) == want, (r, c)
+            y[r, c] = 0.0
+    assert int(torch.count_nonzero(y)) == 0
