@@ -189,8 +189,8 @@ int32_t tl_attention_f32(tl_handle *h, const float *q, const float *k, const flo
 /* TL:159-161 silu (u == NULL) or the GLU product silu(g) * u (GI:212). */
 int32_t tl_silu_mul(tl_handle *h, const float *g, const float *u, int64_t n, float *y);
 /* GQA attention of query rows over sequence seq's INT8 cache at layer:
- * q8 [rows][Hq*64] with per-row scales, row r at position pos0 + r attends
- * keys 0..pos0+r; out [rows][Hq*64] float32 (GI:150-163 with the INT8 score
+ * q8 [rows][Hq*64] with per-row finite scales of either sign, row r at position
+ * pos0 + r attends keys 0..pos0+r; out [rows][Hq*64] float32 (GI:150-163 with the INT8 score
  * and P x V contractions of gemm_operand_router.sv:99-113). */
 int32_t tl_attention(tl_handle *h, int32_t seq, int32_t layer, int32_t pos0, int32_t rows,
                      const int8_t *q8, const double *q_scale, float *out);

@@ -1025,9 +1025,11 @@ TL_DEV double tile_q_scale(const AttnTileArgs& p, int r) {
 // 4 (l / 32) + i % 4 of a 32-key tile), so that a row's scale, maximum, total
 // and last key are one value per lane.  Wavefront w owns the 64-key blocks
 // w, w + NW, ...; scores are recomputed by MFMA in each of three passes.
-//   pass A  each row's largest INT32 score: the score scale is positive, so
-//           f32(S) rs is monotone in S and the maximum of the products is the
-//           product of the maximum (half an instruction per key, v_max3)
+//   pass A  each row's largest INT32 score: f32(S) rs is monotone in S, so the
+//           maximum of the products is the product of the maximum (half an
+//           instruction per key, v_max3).  The quantizer's scales are positive; a
+//           caller's own row scale may be negative, and such a row's scores are
+//           compared inverted (~S falls as S rises), on a branch of its own
 //   pass B  exponentials and block sums (as attention_tile_reg_kernel)
 //   pass C  probabilities and P . V.  rne(127 e / total) is 0 for every key
 //           below a score that follows from the row's maximum and total, and at
@@ -1104,6 +1106,8 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_kernel(AttnTileArgs
     tile_q_frags(p, qs8, col, hi, tq);
     const v4i qa0 = tq.qa0, qa1 = tq.qa1;
     const float rs = scl[col];
+    const int flip = rs < 0.0f ? -1 : 0;
+    const bool any_flip = __any(flip);
     const int rpos = pos_first + col;
     v16i S0, S1;   // scores of the current block's two tiles
     auto scores = [&](int next) {
@@ -1120,6 +1124,12 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_kernel(AttnTileArgs
     int mxs = -2147483647 - 1;
     for (int b = wave; b < nblk; b += NW) {
         scores(b == last ? wave : b + NW);
+        if (any_flip)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                S0[i] ^= flip;
+                S1[i] ^= flip;
+            }
         if (64 * b + 63 <= pos_first) {   // every row sees the whole block
 #pragma unroll
             for (int i = 0; i < 16; i++) mxs = max(mxs, max(S0[i], S1[i]));
@@ -1138,7 +1148,7 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_kernel(AttnTileArgs
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < NW; w++) mxs = max(mxs, wmax[w][col]);
-    const float m = (float)mxs * rs;
+    const float m = (float)(mxs ^ flip) * rs;
 
     // pass B: exponentials and block sums in the butterfly order
     for (int b = wave; b < nblk; b += NW) {
@@ -2185,11 +2195,20 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_reg_kernel(AttnTile
     __syncthreads();
     tile_q_frags(p, qs8, col, hi, tq);
     const float rs = scl[col];
+    const int flip = rs < 0.0f ? -1 : 0;   // as in attention_tile_kernel
+    const bool any_flip = __any(flip);
     const int rpos = pos_first + col, t0 = 64 * wave + 4 * hi;
     const bool whole = 64 * wave + 63 <= pos_first;   // every row sees the whole block
 
     // pass A: scores and each row's largest
     v16i S[2];
+    auto invert = [&]() {
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            S[0][i] ^= flip;
+            S[1][i] ^= flip;
+        }
+    };
     int mxs = -2147483647 - 1;
     if (mine) {
 #pragma unroll
@@ -2197,6 +2216,7 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_reg_kernel(AttnTile
             S[c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[2 * c], tq.qa0, (v16i){}, 0, 0, 0);
             S[c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[2 * c + 1], tq.qa1, S[c], 0, 0, 0);
         }
+        if (any_flip) invert();
         if (whole) {
 #pragma unroll
             for (int i = 0; i < 16; i++) mxs = max(mxs, max(S[0][i], S[1][i]));
@@ -2208,13 +2228,14 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_reg_kernel(AttnTile
                 mxs = t + 32 <= rpos ? max(mxs, S[1][i]) : mxs;
             }
         }
+        if (any_flip) invert();
         mxs = max(mxs, lane_xor<32>(mxs));
     }
     if (hi == 0) wmax[wave][col] = mxs;
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < NW; w++) mxs = max(mxs, wmax[w][col]);
-    const float m = (float)mxs * rs;
+    const float m = (float)(mxs ^ flip) * rs;
 
     // pass B: exponentials (kept) and block sums in the butterfly order
     float ex[2][16];
