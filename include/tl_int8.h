@@ -213,11 +213,13 @@ int32_t tl_lm_head_argmax(tl_handle *h, const float *x, int32_t *token, float *l
 /* Embedding rows for tokens [rows] (dev) into x [rows][D] (dev). */
 int32_t tl_embed(tl_handle *h, const int32_t *tokens, int32_t rows, float *x);
 /* One decoder layer (GI:256-281) for one token of sequence seq at position
- * pos, x [D] dev updated in place, appends the token's K/V rows. */
+ * pos, x [D] dev updated in place, appends the token's K/V rows.  After an
+ * internal error x is undefined (half updated); nothing uses it any more. */
 int32_t tl_decode_layer(tl_handle *h, int32_t seq, int32_t layer, int32_t pos, float *x);
 /* mixed_precision_decoder_layer (GI:256-281) over `rows` consecutive tokens of
  * sequence seq at positions pos0..pos0+rows-1 (causal attention over the
- * cache, whose rows for these positions it writes); x [rows][D] dev in place. */
+ * cache, whose rows for these positions it writes); x [rows][D] dev in place,
+ * undefined after an internal error as in tl_decode_layer. */
 int32_t tl_layer_rows(tl_handle *h, int32_t seq, int32_t layer, int32_t pos0, int32_t rows, float *x);
 /* forward_mixed (GI:437-467) with the quantized LM head: prefill of tokens [n]
  * (host) as tl_prefill, plus the logits of every position into logits, dev

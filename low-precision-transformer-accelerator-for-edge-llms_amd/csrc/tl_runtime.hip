@@ -363,6 +363,17 @@ int32_t finish(tl_handle* h) {
     return TL_OK;
 }
 
+// the result of an entry point whose queued work uses the caller's memory: an
+// error waits for that work (and takes the error it reports out of HIP's state),
+// so that the caller may free the memory on any return
+int32_t drained(tl_handle* h, int32_t r) {
+    if (r != TL_OK) {
+        (void)hipStreamSynchronize(h->stream);
+        (void)hipGetLastError();
+    }
+    return r;
+}
+
 // ---- GEMM dispatch: M == 1 uses the GEMV kernels, M > 1 the MFMA kernels ----
 
 // h->partials of at least `need` elements.  A captured batch step may hold the
@@ -953,7 +964,7 @@ int32_t set_decode_row(tl_handle* h, int32_t seq, int32_t pos, int32_t eos_id) {
 // The single-layer entry points run on the caller's rows in place: the layer's
 // kernels read and write h->x, which is the caller's buffer while this lives.
 // The kernels use 16-byte accesses; an unaligned buffer is copied in and out
-// instead (copy()).
+// instead (copy).
 struct CallerRows {
     tl_handle* h;
     float* own;
@@ -968,6 +979,18 @@ struct CallerRows {
     hipError_t in() const { return copy ? hipMemcpyAsync(own, x, bytes, hipMemcpyDeviceToDevice, h->stream) : hipSuccess; }
     hipError_t out() const { return copy ? hipMemcpyAsync(x, own, bytes, hipMemcpyDeviceToDevice, h->stream) : hipSuccess; }
 };
+
+// one layer over the caller's rows (tl_decode_layer, tl_layer_rows), waited for
+int32_t layer_call(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, int32_t rows, float* x) {
+    int32_t r;
+    set_rows(h, seq, pos0);
+    const CallerRows cx(h, x, rows);
+    TL_HIP(h, cx.in());
+    if (rows > 1 && (r = discard_pending_sums(h))) return r;
+    if ((r = layer_rows(h, layer, rows, pos0 + rows, rows == 1, false))) return r;
+    TL_HIP(h, cx.out());
+    return finish(h);
+}
 
 // clears the abort word when a watched decode or prefill returns (also on an
 // error path), so no later step of another call reads a stale abort
@@ -1677,13 +1700,7 @@ int32_t tl_decode_layer(tl_handle* h, int32_t seq, int32_t layer, int32_t pos, f
     TL_REQ(h, pos >= 0 && pos < c.max_pos, "position out of range");
     TL_REQ(h, x, "null pointer");
     if (!h->layers[layer].wqkv) return fail(h, TL_ERR_BAD_DESCRIPTOR, "layer not loaded");
-    int32_t r;
-    set_rows(h, seq, pos);
-    const CallerRows cx(h, x, 1);
-    TL_HIP(h, cx.in());
-    if ((r = layer_rows(h, layer, 1, pos + 1, true, false))) return r;
-    TL_HIP(h, cx.out());
-    return finish(h);
+    return drained(h, layer_call(h, seq, layer, pos, 1, x));
 }
 
 }  // extern "C"
@@ -1739,6 +1756,7 @@ int32_t prefill_layers(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t
 }
 
 // next-token bookkeeping from the last prompt row, then wait and report
+// (with an error, work on the caller's tokens may be left queued)
 int32_t prefill_finish(tl_handle* h, int32_t seq, int32_t n, int32_t* next_token, float* next_logit) {
     const tl_config& c = h->cfg;
     int32_t r;
@@ -1758,13 +1776,15 @@ extern "C" {
 int32_t tl_prefill(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t n, int32_t* next_token, float* next_logit) {
     if (!h) return TL_ERR_BAD_DESCRIPTOR;
     int32_t r = prefill_layers(h, seq, tokens, n);
-    if (r) return r;
-    return prefill_finish(h, seq, n, next_token, next_logit);
+    if (!r) r = prefill_finish(h, seq, n, next_token, next_logit);
+    return drained(h, r);
 }
 
-int32_t tl_prefill_logits(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t n, float* logits) {
-    if (!h) return TL_ERR_BAD_DESCRIPTOR;
-    TL_REQ(h, logits, "null pointer");
+}  // extern "C"
+
+namespace {
+
+int32_t prefill_logits(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t n, float* logits) {
     int32_t r = prefill_layers(h, seq, tokens, n);
     if (r) return r;
     const tl_config& c = h->cfg;
@@ -1779,6 +1799,16 @@ int32_t tl_prefill_logits(tl_handle* h, int32_t seq, const int32_t* tokens, int3
     return prefill_finish(h, seq, n, nullptr, nullptr);
 }
 
+}  // namespace
+
+extern "C" {
+
+int32_t tl_prefill_logits(tl_handle* h, int32_t seq, const int32_t* tokens, int32_t n, float* logits) {
+    if (!h) return TL_ERR_BAD_DESCRIPTOR;
+    TL_REQ(h, logits, "null pointer");
+    return drained(h, prefill_logits(h, seq, tokens, n, logits));
+}
+
 int32_t tl_layer_rows(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, int32_t rows, float* x) {
     if (!h) return TL_ERR_BAD_DESCRIPTOR;
     const tl_config& c = h->cfg;
@@ -1787,14 +1817,7 @@ int32_t tl_layer_rows(tl_handle* h, int32_t seq, int32_t layer, int32_t pos0, in
     TL_REQ(h, pos0 >= 0 && (int64_t)pos0 + rows <= c.max_pos, "Sequence length exceeds max_position_embeddings");
     TL_REQ(h, x, "null pointer");
     if (!h->layers[layer].wqkv) return fail(h, TL_ERR_BAD_DESCRIPTOR, "layer not loaded");
-    int32_t r;
-    set_rows(h, seq, pos0);
-    const CallerRows cx(h, x, rows);
-    TL_HIP(h, cx.in());
-    if (rows > 1 && (r = discard_pending_sums(h))) return r;
-    if ((r = layer_rows(h, layer, rows, pos0 + rows, rows == 1, false))) return r;
-    TL_HIP(h, cx.out());
-    return finish(h);
+    return drained(h, layer_call(h, seq, layer, pos0, rows, x));
 }
 
 int32_t tl_dequantize_i32(tl_handle* h, const int32_t* acc, int64_t rows, int32_t cols, double input_scale,
@@ -1907,12 +1930,12 @@ int32_t tl_generate(tl_handle* h, int32_t seq, const int32_t* prompt, int32_t n_
     int32_t first = 0;
     bool aborted = false;
     int32_t r = prefill_layers(h, seq, prompt, n_prompt, abort_flag, &aborted);
-    if (r) return r;
+    if (r) return drained(h, r);
     if (aborted) {
         if (stop_reason) *stop_reason = TL_STOP_HOST_ABORT;
         return TL_OK;
     }
-    if ((r = prefill_finish(h, seq, n_prompt, &first, nullptr))) return r;
+    if ((r = prefill_finish(h, seq, n_prompt, &first, nullptr))) return drained(h, r);
     tokens_out[0] = first;
     *n_out = 1;
     if (eos_id >= 0 && first == eos_id) {
