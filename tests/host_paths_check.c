@@ -5,7 +5,9 @@
  * the host's, kernels are counted and not run, work on a stream is "queued"
  * until the next hipStreamSynchronize, and the operation number fail_at (a
  * launch or an asynchronous copy) returns an error.  A failing call must not
- * return with work still queued that reads or writes the caller's memory.
+ * return with work still queued that reads or writes the caller's memory.  A
+ * captured step may hold the address of any buffer that was there when it was
+ * instantiated: none may be launched after such a buffer was freed.
  *
  * Built with -rdynamic and linked with the library; prints one line per
  * scenario and exits with the number of violations. */
@@ -27,6 +29,13 @@ static hipError_t op(void) {
     return hipSuccess;
 }
 
+/* device buffers and captured steps, by order of birth */
+enum { MAXBUF = 1024, MAXEXEC = 64 };
+static struct { void* p; long born; } bufs[MAXBUF];
+static struct exec { long born; int stale; } *execs[MAXEXEC];
+static long births;
+static int stale_launches;
+
 /* ---- the HIP entry points the library uses --------------------------------- */
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
@@ -39,8 +48,27 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int d) {
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int d) { (void)a; (void)d; *v = 256; return hipSuccess; }
 const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "ok" : "planted failure"; }
 hipError_t hipGetLastError(void) { hipError_t e = last; last = hipSuccess; return e; }
-hipError_t hipMalloc(void** p, size_t n) { *p = aligned_alloc(256, (n + 255) / 256 * 256); return *p ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n) {
+    *p = aligned_alloc(256, (n + 255) / 256 * 256);
+    for (int i = 0; *p && i < MAXBUF; i++)
+        if (!bufs[i].p) {
+            bufs[i].p = *p;
+            bufs[i].born = ++births;
+            return hipSuccess;
+        }
+    return hipErrorOutOfMemory;
+}
+hipError_t hipFree(void* p) {
+    for (int i = 0; p && i < MAXBUF; i++)
+        if (bufs[i].p == p) {
+            for (int j = 0; j < MAXEXEC; j++)
+                if (execs[j] && execs[j]->born > bufs[i].born) execs[j]->stale = 1;
+            bufs[i].p = NULL;
+            break;
+        }
+    free(p);
+    return hipSuccess;
+}
 hipError_t hipHostMalloc(void** p, size_t n, unsigned f) { (void)f; *p = calloc(1, n); return hipSuccess; }
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned f) { (void)f; *d = h; return hipSuccess; }
@@ -68,12 +96,28 @@ hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode m) { (void)
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) { (void)s; capturing = 0; *g = (hipGraph_t)1; return hipSuccess; }
 hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t g, hipGraphNode_t* n, char* b, size_t z) {
     (void)g; (void)n; (void)b; (void)z;
-    *x = (hipGraphExec_t)malloc(1);
-    return hipSuccess;
+    for (int j = 0; j < MAXEXEC; j++)
+        if (!execs[j]) {
+            execs[j] = malloc(sizeof(struct exec));
+            execs[j]->born = ++births;
+            execs[j]->stale = 0;
+            *x = (hipGraphExec_t)execs[j];
+            return hipSuccess;
+        }
+    return hipErrorOutOfMemory;
 }
 hipError_t hipGraphDestroy(hipGraph_t g) { (void)g; return hipSuccess; }
-hipError_t hipGraphExecDestroy(hipGraphExec_t x) { free(x); return hipSuccess; }
-hipError_t hipGraphLaunch(hipGraphExec_t x, hipStream_t s) { (void)x; (void)s; return op(); }
+hipError_t hipGraphExecDestroy(hipGraphExec_t x) {
+    for (int j = 0; j < MAXEXEC; j++)
+        if ((void*)execs[j] == (void*)x) execs[j] = NULL;
+    free(x);
+    return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t x, hipStream_t s) {
+    (void)s;
+    stale_launches += ((struct exec*)x)->stale;
+    return op();
+}
 static dim3 cfg_grid, cfg_block;
 static size_t cfg_lds;
 static hipStream_t cfg_stream;
@@ -91,12 +135,12 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** a, size_t l, hi
 }
 
 /* ---- a small model and the calls -------------------------------------------- */
-enum { D = 512, F = 1024, HKV = 2, V = 256, MAXPOS = 256, LAYERS = 2 };
+enum { D = 512, HKV = 2, V = 256, MAXPOS = 256, LAYERS = 2 };
 
-static tl_handle* make(void) {
+static tl_handle* make(int F, int max_seqs) {
     const tl_config c = {D, F, LAYERS, D / 64, HKV, 64, V, MAXPOS, 1e-5f, 10000.0f};
     tl_handle* h = NULL;
-    if (tl_create(&c, 4, &h) != TL_OK) {
+    if (tl_create(&c, max_seqs, &h) != TL_OK) {
         printf("tl_create: %s\n", tl_last_error(NULL));
         exit(100);
     }
@@ -131,6 +175,21 @@ static int run(tl_handle* h, const struct call* c) {
     return tl_generate(h, 0, tokens, c->n, 1, -1, NULL, &tok, &n, NULL);
 }
 
+/* batches whose split-K scratch grows (1408 is no multiple of 512: no packed
+ * form), back to the small ones, on one handle */
+static int alternating_batches(void) {
+    static const int sizes[] = {4, 40, 60, 0, 4, 40, 60};   /* 0: a scored prompt of 63 tokens */
+    static int32_t start[60], out[60 * 4];
+    tl_handle* h = make(1408, 60);
+    int wrong = 0;
+    for (size_t i = 0; i < sizeof sizes / sizeof sizes[0]; i++)
+        wrong += (sizes[i] ? tl_decode_batch(h, sizes[i], tokens, start, 4, out)
+                           : tl_prefill_logits(h, 0, tokens, 63, logits)) != TL_OK;
+    printf("alternating batches: %d failed, %d launches of steps that hold a freed buffer\n", wrong, stale_launches);
+    tl_destroy(h);
+    return wrong + stale_launches;
+}
+
 int main(void) {
     static const struct call calls[] = {
         {"layer", 1, 0}, {"layer", 1, 1}, {"rows", 1, 0}, {"rows", 5, 0}, {"rows", 5, 3}, {"rows", 40, 0}, {"rows", 70, 0},
@@ -141,7 +200,7 @@ int main(void) {
     int bad = 0;
     for (size_t i = 0; i < sizeof calls / sizeof calls[0]; i++) {
         const struct call* c = &calls[i];
-        tl_handle* h = make();
+        tl_handle* h = make(1024, 4);
         ops = fail_at = 0;
         int wrong = run(h, c) != TL_OK || queued != 0;
         const long total = ops;
@@ -159,5 +218,6 @@ int main(void) {
         tl_destroy(h);
     }
     free(rows);
+    bad += alternating_batches();
     return bad > 255 ? 255 : bad;
 }
