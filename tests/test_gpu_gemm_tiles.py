@@ -22,10 +22,10 @@ def rt():
     (2048, 2048, 128),    # 128 x 128 tiles, one round, two 64-byte stages
     (1999, 2017, 256),    # ... ragged rows and columns
     (1999, 2081, 256),    # five rounds of 64 x 64 tiles against two: 64 x 64, ragged
-    (65, 32000, 128),     # ... the second row half of every tile nearly empty
+    (65, 32000, 128),     # 128 x 128, the second row half of every tile nearly empty
     (2048, 2560, 384),    # just below the rule: 64 x 64 tiles
     (1100, 2048, 128),    # three rounds against one: 64 x 64
-    (333, 9000, 1152),
+    (333, 9000, 1152),    # 128 x 128, one ragged round
     (64, 64, 128),
 ])
 def test_gemm_tile_sizes(rt, m, n, k):
@@ -53,11 +53,23 @@ def test_gemm_tile_sizes(rt, m, n, k):
     assert_bits_equal(host(y), res + deq, "with residual")
 
 
-@pytest.mark.parametrize("B,vocab", [(33, 2048), (40, 32000), (129, 24000)])
-def test_many_row_lm_head_ties(B, vocab):
+def _large_tiles(m, n):
+    """The size rule of the row-major tiles: 128 x 128 where 64 x 64 ones need at
+    least four rounds of the 256 CUs, and three for each round of theirs."""
+    r64, r128 = (-(-(-(-n // t) * -(-m // t)) // 256) for t in (64, 128))
+    return r64 >= 4 and r64 >= 3 * r128
+
+
+@pytest.mark.parametrize("B,vocab,large", [
+    (33, 2048, False), (40, 32000, False), (129, 24000, False),   # 1, 2 and 5 rounds (5 against 2)
+    (65, 32000, True), (90, 32000, True),                         # 4 rounds against 1
+    (129, 32000, True),                                           # 6 against 2, one row in the second row tile
+])
+def test_many_row_lm_head_ties(B, vocab, large):
     """The LM head over more than 32 rows takes the argmax in its tiles: with
     every head row repeated once in the same 32 columns and once far away, equal
-    logits resolve to the lowest id, for both tile sizes."""
+    logits resolve to the lowest id, in 64 x 64 and in 128 x 128 tiles."""
+    assert _large_tiles(B, vocab) == large
     from lpta.engine import Engine
     cfg = dict(oracle.SMALL_CFG, n_layers=1, vocab=vocab)
     m = oracle.synthetic_model(cfg, seed=B)
