@@ -108,7 +108,7 @@ def layer_eng():
     e.close()
 
 
-@pytest.mark.parametrize("rows", [32, 33, 63, 64, 65, 128, 129, 256, 257, 300])
+@pytest.mark.parametrize("rows", [32, 33, 63, 64, 65, 128, 129, 256, 257, 300, 384, 385])
 def test_layer_rows_equal_single_rows(layer_eng, rows):
     """Both sides of every row count at which a projection changes kernel: the
     layer over all rows equals the single-row kernels run row after row on
