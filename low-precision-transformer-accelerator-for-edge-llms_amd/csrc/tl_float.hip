@@ -6,6 +6,9 @@
 // reference to float32 rounding, not bit for bit.  Not on the INT8 hot path.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "tl_device.h"
 #include "tl_internal.h"
 
@@ -25,39 +28,53 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 // What bounds it: the float32 matrix rate at hundreds of rows (640 x 5632 x
 // 2048: 90 TFLOP/s; 100 x 5632 x 2048 puts 236 of 256 CUs at work), launch and
 // latency at a few.  The whole call at 100 x 5632 x 2048: 245 us with 64 x 64 vector-FMA
-// tiles through LDS, 51 us now; 640 rows 407 -> 167; one row 238 -> 28.  Eight
+// tiles through LDS, 50 us now; 640 rows 407 -> 170; one row 238 -> 28.  Eight
 // partial sums per output also round less: 2.9e-7 relative to 64 bits where
 // one chain of 2048 had 8.1e-7.
 constexpr int kLinWaves = 8;
 
-// OFF: unsigned lane offsets of elements, or int64_t where 32 k or 8 n passes 2^32
-template <int NB, bool VEC, typename OFF>
+// WIDE: the form for every size.  The other one counts tiles in one grid
+// dimension and lane offsets and columns in 32 bits (launch_linear_f32 says up to
+// where); its shorter start is worth 0.5-0.7 us of a whole call (38.3 against 39.0 us
+// at 33 x 5632 x 2048, 50.3 against 51.0 at 100 rows).
+template <int NB, bool VEC, bool WIDE>
 __global__ __launch_bounds__(kLinWaves * 64) void linear_f32_kernel(const float* __restrict__ x,
                                                                     const float* __restrict__ w,
                                                                     const float* __restrict__ b,
                                                                     const float* __restrict__ residual, int32_t m,
-                                                                    int32_t n, int32_t k, int32_t tiles_n,
-                                                                    float* __restrict__ y) {
+                                                                    int32_t n, int32_t k, int32_t tiles_m,
+                                                                    int32_t tiles_n, float* __restrict__ y) {
+    using Off = std::conditional_t<WIDE, int64_t, unsigned>;
+    using Col = std::conditional_t<WIDE, unsigned, int>;   // the last tile's columns may pass 2^31
     constexpr int PD = NB == 1 ? 8 : 4, HW = kLinWaves / 2;   // chunks in flight; LDS partial tiles
     __shared__ float red[HW][NB * 16][64];
-    // workgroups go to the 8 XCDs round-robin in x (8 x the row tiles), y, z order: the
-    // row tiles of a column tile stay on one XCD, whose L2 then holds the column
-    // tile's weights
-    const int tm = (int)blockIdx.x >> 3, tn = (int)(blockIdx.z * gridDim.y + blockIdx.y) * 8 + ((int)blockIdx.x & 7);
+    // workgroups go to the 8 XCDs round-robin: the row tiles of a column tile
+    // stay on one XCD, whose L2 then holds the column tile's weights.  One
+    // dimension, or (wide) 8 x the row tiles in x and groups of 8 column tiles in y
+    // and z: the same order
+    int tm, tn;
+    if constexpr (WIDE) {
+        tm = (int)blockIdx.x >> 3;
+        tn = (int)(blockIdx.z * gridDim.y + blockIdx.y) * 8 + ((int)blockIdx.x & 7);
+    } else {
+        const int q = (int)blockIdx.x >> 3;
+        tn = q / tiles_m * 8 + ((int)blockIdx.x & 7);
+        tm = q % tiles_m;
+    }
     if (tn >= tiles_n) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), col = lane & 31, hi = lane >> 5;
     const int64_t row0 = (int64_t)tm * 32;
-    const unsigned col0 = (unsigned)tn * 32 * NB;   // column indices pass 2^31 in the last tile of the widest n
-    const int nfull = k >> 3, nch = nfull + ((k & 7) != 0), per = (nch + kLinWaves - 1) / kLinWaves;
+    const Col col0 = (Col)tn * 32 * NB;
+    const int nfull = k >> 3, nch = WIDE ? nfull + ((k & 7) != 0) : (k + 7) >> 3, per = (nch + kLinWaves - 1) / kLinWaves;
     const int c0 = min(wave * per, nfull), c1 = min(c0 + per, nfull);   // this wavefront's whole chunks
     // one wavefront-uniform base per chunk, and lane offsets formed once
     const float* xb = x + row0 * k;
-    const OFF xo = (OFF)min(col, (int)(m - 1 - row0)) * (OFF)k + 4 * hi;
-    OFF wo[4][NB];
+    const Off xo = (Off)min(col, (int)(m - 1 - row0)) * (Off)k + 4 * hi;
+    Off wo[4][NB];
 #pragma unroll
     for (int s = 0; s < 4; s++)
 #pragma unroll
-        for (int j = 0; j < NB; j++) wo[s][j] = (OFF)(4 * hi + s) * (OFF)n + min(col0 + 32 * j + col, (unsigned)n - 1);
+        for (int j = 0; j < NB; j++) wo[s][j] = (Off)(4 * hi + s) * (Off)n + (unsigned)min(col0 + 32 * j + col, (Col)n - 1);
     v16f acc[NB];
 #pragma unroll
     for (int j = 0; j < NB; j++) acc[j] = (v16f){};
@@ -131,8 +148,8 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_f32_kernel(const float*
     for (int i = 0; i < 2 * NB; i++) {   // output register e of block j: 16 NB of them over 8 wavefronts
         const int je = i * kLinWaves + wave, e = je & 15;
         const int64_t r = row0 + 8 * (e >> 2) + 4 * hi + (e & 3);
-        const unsigned c = col0 + 32 * (je >> 4) + col;
-        if (r >= m || c >= (unsigned)n) continue;
+        const Col c = col0 + 32 * (je >> 4) + col;
+        if (r >= m || c >= (Col)n) continue;
         float v = (red[0][je][lane] + red[1][je][lane]) + (red[2][je][lane] + red[3][je][lane]);
         if (b) v = v + b[c];
         const int64_t idx = r * n + c;
@@ -141,23 +158,21 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_f32_kernel(const float*
     }
 }
 
-template <int NB, bool VEC, typename OFF>
-void go_linear_kernel(hipStream_t s, const float* x, const float* w, const float* b, const float* residual, int32_t m,
-                      int32_t n, int32_t k, float* y) {
-    // three grid dimensions: one would pass the limit of 2^32 threads at 8.4 million tiles
-    constexpr int32_t kMaxY = 32768;
-    const int32_t tm = (int32_t)(((int64_t)m + 31) / 32), tn = (int32_t)(((int64_t)n + 32 * NB - 1) / (32 * NB));
-    const int32_t cols8 = (tn + 7) / 8;   // groups of 8 column tiles, one per XCD
-    const dim3 grid(8u * (unsigned)tm, std::min(cols8, kMaxY), (cols8 + kMaxY - 1) / kMaxY);
-    TL_KLAUNCH((linear_f32_kernel<NB, VEC, OFF>), grid, dim3(kLinWaves * 64), 0, s, x, w, b, residual, m, n, k, tn, y);
-}
-
 template <int NB>
 void go_linear(hipStream_t s, const float* x, const float* w, const float* b, const float* residual, int32_t m,
-               int32_t n, int32_t k, float* y) {
+               int32_t n, int32_t k, int32_t tm, int32_t tn, float* y) {
+    const dim3 grid((unsigned)((tn + 7) / 8 * 8) * (unsigned)tm), block(kLinWaves * 64);
     if (k % 4 == 0 && (uintptr_t)x % 16 == 0)
-        go_linear_kernel<NB, true, unsigned>(s, x, w, b, residual, m, n, k, y);
-    else go_linear_kernel<NB, false, unsigned>(s, x, w, b, residual, m, n, k, y);
+        TL_KLAUNCH((linear_f32_kernel<NB, true, false>), grid, block, 0, s, x, w, b, residual, m, n, k, tm, tn, y);
+    else TL_KLAUNCH((linear_f32_kernel<NB, false, false>), grid, block, 0, s, x, w, b, residual, m, n, k, tm, tn, y);
+}
+
+void go_linear_wide(hipStream_t s, const float* x, const float* w, const float* b, const float* residual, int32_t m,
+                    int32_t n, int32_t k, float* y) {
+    constexpr int32_t kMaxY = 32768;
+    const int32_t tm = (int32_t)(((int64_t)m + 31) / 32), tn = (int32_t)(((int64_t)n + 31) / 32), g = (tn + 7) / 8;
+    const dim3 grid(8u * (unsigned)tm, std::min(g, kMaxY), (g + kMaxY - 1) / kMaxY), block(kLinWaves * 64);
+    TL_KLAUNCH((linear_f32_kernel<1, false, true>), grid, block, 0, s, x, w, b, residual, m, n, k, tm, tn, y);
 }
 
 // one (query row i, query head h) per workgroup; the row's scores live in LDS
@@ -232,27 +247,31 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
 hipError_t launch_linear_f32(hipStream_t s, const float* x, const float* w, const float* b, const float* residual,
                              int32_t m, int32_t n, int32_t k, float* y) {
     if (m <= 0 || n <= 0) return hipSuccess;
-    if (k >= 1 << 27 || n > 1 << 29) {   // lane offsets past 2^32
-        go_linear_kernel<1, false, int64_t>(s, x, w, b, residual, m, n, k, y);
-        return hipGetLastError();
-    }
     // column blocks per tile: the fewest MFMAs on the busiest CU (rounds of 256
     // tiles times blocks); of equals the widest, which reads x least often
     const int64_t tm = ((int64_t)m + 31) / 32;
     int nb = 1;
-    int64_t best = INT64_MAX;
+    int64_t best = INT64_MAX, tn = 0;
     for (int c = 1; c <= 4; c++) {
-        const int64_t cost = (tm * (((int64_t)n + 32 * c - 1) / (32 * c)) + 255) / 256 * c;
+        const int64_t t = ((int64_t)n + 32 * c - 1) / (32 * c), cost = (tm * t + 255) / 256 * c;
         if (cost <= best) {
             best = cost;
             nb = c;
+            tn = t;
         }
     }
+    // offsets inside a tile below 2^32 (31 k + 8 and 8 n), and a grid below 2^32
+    // threads of one dimension
+    if (k >= 1 << 27 || n > 1 << 29 || (tn + 7) / 8 * 8 * tm >= 1 << 23) {
+        go_linear_wide(s, x, w, b, residual, m, n, k, y);
+        return hipGetLastError();
+    }
+    const int32_t m32 = (int32_t)tm, n32 = (int32_t)tn;
     switch (nb) {
-        case 1: go_linear<1>(s, x, w, b, residual, m, n, k, y); break;
-        case 2: go_linear<2>(s, x, w, b, residual, m, n, k, y); break;
-        case 3: go_linear<3>(s, x, w, b, residual, m, n, k, y); break;
-        default: go_linear<4>(s, x, w, b, residual, m, n, k, y); break;
+        case 1: go_linear<1>(s, x, w, b, residual, m, n, k, m32, n32, y); break;
+        case 2: go_linear<2>(s, x, w, b, residual, m, n, k, m32, n32, y); break;
+        case 3: go_linear<3>(s, x, w, b, residual, m, n, k, m32, n32, y); break;
+        default: go_linear<4>(s, x, w, b, residual, m, n, k, m32, n32, y); break;
     }
     return hipGetLastError();
 }

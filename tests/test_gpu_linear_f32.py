@@ -92,3 +92,21 @@ def test_linear_f32_offsets_past_32_bits(rt, m, n, k):
             assert float(y[r, c]) == want, (r, c)
             y[r, c] = 0.0
     assert int(torch.count_nonzero(y)) == 0
+    del x, w, y
+    torch.cuda.empty_cache()
+
+
+def test_linear_f32_tiles_past_one_grid_dimension(rt):
+    """8.4 million tiles of 512 threads, 2^32 threads in one dimension: an
+    outer product of small whole numbers, every element compared."""
+    import torch
+    m, n = 16_777_300, 800   # 524291 row tiles x 9 column tiles of 96, counted as 16
+    x = (torch.arange(m, device="cuda") % 251).float().reshape(m, 1)
+    w = (torch.arange(n, device="cuda") % 13 + 1).float().reshape(1, n)
+    y = torch.empty((m, n), device="cuda")
+    torch.cuda.synchronize()
+    rt.call("tl_linear_f32", x, w, None, None, m, n, 1, y)
+    for i in range(0, m, 1 << 21):
+        assert torch.equal(y[i:i + (1 << 21)], x[i:i + (1 << 21)] * w), i
+    del x, w, y
+    torch.cuda.empty_cache()
