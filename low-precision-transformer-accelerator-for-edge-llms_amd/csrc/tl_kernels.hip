@@ -1027,9 +1027,9 @@ TL_DEV double tile_q_scale(const AttnTileArgs& p, int r) {
 // w, w + NW, ...; scores are recomputed by MFMA in each of three passes.
 //   pass A  each row's largest INT32 score: f32(S) rs is monotone in S, so the
 //           maximum of the products is the product of the maximum (half an
-//           instruction per key, v_max3).  The quantizer's scales are positive; a
-//           caller's own row scale may be negative, and such a row's scores are
-//           compared inverted (~S falls as S rises), on a branch of its own
+//           instruction per key, v_max3).  The quantizer's scales are positive;
+//           those a caller brings with INT8 Q may be negative (SIGNED), and such a
+//           row's scores are compared inverted: ~S falls as S rises
 //   pass B  exponentials and block sums (as attention_tile_reg_kernel)
 //   pass C  probabilities and P . V.  rne(127 e / total) is 0 for every key
 //           below a score that follows from the row's maximum and total, and at
@@ -1064,7 +1064,7 @@ TL_DEV v4i prob_frag(const unsigned* w) {
     return (v4i){(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
 }
 
-template <int NW>
+template <int NW, bool SIGNED>
 __global__ __launch_bounds__(NW * 64, 4) void attention_tile_kernel(AttnTileArgs p) {
     extern __shared__ __align__(16) int8_t tile_lds[];
     __shared__ __align__(16) int8_t qs8[32 * 64];   // Q quantized by the workgroup (float32 Q input)
@@ -1106,8 +1106,8 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_kernel(AttnTileArgs
     tile_q_frags(p, qs8, col, hi, tq);
     const v4i qa0 = tq.qa0, qa1 = tq.qa1;
     const float rs = scl[col];
-    const int flip = rs < 0.0f ? -1 : 0;
-    const bool any_flip = __any(flip);
+    const int flip = SIGNED && rs < 0.0f ? -1 : 0;
+    const bool any_flip = SIGNED && __any(flip);
     const int rpos = pos_first + col;
     v16i S0, S1;   // scores of the current block's two tiles
     auto scores = [&](int next) {
@@ -2163,7 +2163,7 @@ static size_t tile_lds_bytes(int nblk) { return (size_t)32 * 64 * sizeof(int) + 
 // crosses lanes, the others add registers of one lane.  512 rows from key 0:
 // 12.4 us per launch with one block per wavefront (8 wavefronts), where 4
 // wavefronts of two blocks and probabilities through LDS took 13.9.
-template <int NW>
+template <int NW, bool SIGNED>
 __global__ __launch_bounds__(NW * 64, 4) void attention_tile_reg_kernel(AttnTileArgs p) {
     __shared__ int accs[32 * 64];
     __shared__ __align__(16) float bsum[32 * (NW + 1)];   // an odd row stride spreads the rows over the banks
@@ -2195,8 +2195,8 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_tile_reg_kernel(AttnTile
     __syncthreads();
     tile_q_frags(p, qs8, col, hi, tq);
     const float rs = scl[col];
-    const int flip = rs < 0.0f ? -1 : 0;   // as in attention_tile_kernel
-    const bool any_flip = __any(flip);
+    const int flip = SIGNED && rs < 0.0f ? -1 : 0;   // as in attention_tile_kernel
+    const bool any_flip = SIGNED && __any(flip);
     const int rpos = pos_first + col, t0 = 64 * wave + 4 * hi;
     const bool whole = 64 * wave + 63 <= pos_first;   // every row sees the whole block
 
@@ -2339,12 +2339,18 @@ hipError_t launch_attention_tiles(hipStream_t s, const int8_t* q8, const double*
     // 74.0 against 81.8).
     const int wgs = n_heads * (int)grid.y;
     const size_t lds = tile_lds_bytes(tpad / 64);
-    if (tpad <= 256) TL_KLAUNCH(attention_tile_reg_kernel<4>, grid, block, 0, s, a);
-    else if (tpad <= 512) TL_KLAUNCH(attention_tile_reg_kernel<8>, grid, dim3(512), 0, s, a);
-    else if (tpad <= 1024 && wgs <= 256) TL_KLAUNCH(attention_tile_reg_kernel<16>, grid, dim3(1024), 0, s, a);
-    else if (wgs <= 256) TL_KLAUNCH(attention_tile_kernel<16>, grid, dim3(1024), lds, s, a);
-    else if (wgs < 1024) TL_KLAUNCH(attention_tile_kernel<8>, grid, dim3(512), lds, s, a);
-    else TL_KLAUNCH(attention_tile_kernel<4>, grid, block, lds, s, a);
+    // quantized from float32 Q here: positive scales
+    auto go = [&](auto sgn) {
+        constexpr bool SG = decltype(sgn)::value;
+        if (tpad <= 256) TL_KLAUNCH((attention_tile_reg_kernel<4, SG>), grid, block, 0, s, a);
+        else if (tpad <= 512) TL_KLAUNCH((attention_tile_reg_kernel<8, SG>), grid, dim3(512), 0, s, a);
+        else if (tpad <= 1024 && wgs <= 256) TL_KLAUNCH((attention_tile_reg_kernel<16, SG>), grid, dim3(1024), 0, s, a);
+        else if (wgs <= 256) TL_KLAUNCH((attention_tile_kernel<16, SG>), grid, dim3(1024), lds, s, a);
+        else if (wgs < 1024) TL_KLAUNCH((attention_tile_kernel<8, SG>), grid, dim3(512), lds, s, a);
+        else TL_KLAUNCH((attention_tile_kernel<4, SG>), grid, block, lds, s, a);
+    };
+    if (qf) go(std::false_type{});
+    else go(std::true_type{});
     return hipGetLastError();
 }
 
