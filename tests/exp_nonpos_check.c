@@ -1,6 +1,6 @@
 // The softmax exponential of the GPU kernels (csrc/tl_device.h,
-// tl_expf_nonpos) against the exponential it replaces there (tl_expf_sel,
-// the oracle's tl_expf without branches), bit for bit over every float x in
+// tl_expf_nonpos) against the exponential it replaces there (the oracle's
+// tl_expf, here without branches), bit for bit over every float x in
 // [-90, -0]: the same Cody-Waite reduction and degree-7 polynomial, but no
 // clamp of x to [-80, 80] before the reduction and 2^k applied by ldexp
 // instead of a multiply by the power of two built in the exponent field.

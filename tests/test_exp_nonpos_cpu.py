@@ -1,6 +1,6 @@
 """The GPU softmax exponential for non-positive arguments (tl_device.h
 tl_expf_nonpos: no clamps, 2^k by ldexp) equals the exponential the oracle
-and the other kernels use (tl_expf, branch-free as tl_expf_sel) on every
+and the other kernels use (tl_expf, written without branches) on every
 float in [-90, -0]: the same operation sequence in C (fmaf), compared bit for
 bit, the range below the cut-off at -80 included."""
 import os
