@@ -503,8 +503,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(GemmArgs a) {
         }
 }
 
-// Row-major operands (the tl_gemm_i8 operators, the LM head over many rows and
-// prefill shapes the packed path does not take), M >= 64, 32x32x32 MFMA tiles:
+// Row-major operands (the tl_gemm_i8 operators and prefill shapes the packed
+// path does not take from 64 rows, the LM head from 33), 32x32x32 MFMA tiles:
 //   gemm_tile_kernel, K a multiple of 128: 2 x 2 wavefronts of one 32 x 32
 //     block each (64 x 64 block tile), 128-byte K stages through two LDS
 //     buffers, four register sets; or of 2 x 2 blocks each (128 x 128 block
@@ -550,8 +550,8 @@ static bool shape32(hipStream_t s, const GemmArgs& a, bool tile) {
     return true;
 }
 
-// M >= 64, row-major operands, the whole K in one launch: gemm_tile_kernel
-// (tile; K a multiple of 128) or gemm32_kernel
+// any M (callers come from 64 rows, EPI_ARGMAX from 33), row-major operands, the
+// whole K in one launch: gemm_tile_kernel (tile; K a multiple of 128) or gemm32_kernel
 hipError_t launch_gemm32(hipStream_t s, int epi, const GemmArgs& args, bool tile) {
     GemmArgs a = args;
     if (a.m <= 0 || a.n <= 0) return hipSuccess;

@@ -1641,7 +1641,8 @@ hipError_t launch_argmax_tiles(hipStream_t s, const unsigned long long* part, in
     return hipGetLastError();
 }
 
-// batched decode: the position of each row is its sequence's cursor
+// RowsInit: row r at position pos0 + r of sequence seq (or of seq + r), and one
+// sequence's state where the pointers are given
 __global__ __launch_bounds__(256) void rows_init_kernel(RowsInit a) {
     const int r = blockIdx.x * 256 + threadIdx.x;
     if (r < a.rows) {
@@ -1656,6 +1657,7 @@ __global__ __launch_bounds__(256) void rows_init_kernel(RowsInit a) {
     if (a.stopped) *a.stopped = 0;
 }
 
+// logical [n][64] rows <-> cache plane layout
 __global__ void kv_scatter_kernel(KvGeom kv, int64_t pl, int32_t t0, int32_t n,
                                   const int8_t* __restrict__ k_rows, const int8_t* __restrict__ v_rows) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -570,8 +570,8 @@ GemvArgs gemv_args(const tl_handle* h) {
 }
 
 // one decoder layer (GI:256-281) for a single row (batch-1 decode or a
-// one-token prefill) as five fused kernels; the row's sequence and position
-// are in h->row_seq[0] / h->row_pos[0]; max_t bounds pos + 1
+// one-token prefill) as five fused kernels; the row's sequence and position are
+// given by rowmap(h); max_t bounds pos + 1
 int32_t layer_row1(tl_handle* h, int32_t layer, int32_t max_t) {
     const tl_config& c = h->cfg;
     const LayerDev& L = h->layers[layer];
@@ -713,7 +713,7 @@ static int32_t rows_rmsnorm(tl_handle* h, int32_t rows, const float* g, bool pk 
 }
 
 // one decoder layer (GI:256-281) for `rows` rows of h->x whose sequence and
-// position are in h->row_seq / h->row_pos; max_t bounds pos + 1 over the rows.
+// position are given by rowmap(h); max_t bounds pos + 1 over the rows.
 // decode: every row is a different sequence (its own K/V row is appended by
 // the attention kernel); otherwise the rows are consecutive prompt positions
 // of one sequence (all appended before attention reads them).  The caller has
@@ -891,7 +891,7 @@ int32_t lm_head_rows(tl_handle* h, const float* xrow, int32_t rows, int32_t seq,
         Prof p(h, TL_K_LMHEAD, (double)V * D + V * 4.0 + D * 8.0);
         TL_LAUNCH(h, launch_gemv_fused(h->stream, PRO_RMSNORM, EPI_ARGMAX, g));
     } else {
-        // past 32 rows: row-major tiles with the argmax in their epilogue
+        // past 32 rows: row-major tiles (launch_gemm32) with the argmax in their epilogue
         const bool lm_tile = rows > 32 && D % 128 == 0 && V % 32 == 0;
         if (h->racc_res_ws && xrow == h->x) {
             int32_t r = rows_rmsnorm(h, rows, h->g_final);
@@ -1643,7 +1643,7 @@ int32_t tl_lm_head_argmax(tl_handle* h, const float* x, int32_t* token, float* l
     if ((uintptr_t)x % 16 == 0 && n_wg > 0 && n_wg <= (V + 3) / 4) {
         // the decode step's fused RMSNorm + LM head; its workgroups store their
         // best keys straight into pinned host memory, which is folded here once the
-        // kernel has ended (57 -> 31 us per call against a norm kernel, a GEMV with one
+        // kernel has ended (57 -> 27 us per call against a norm kernel, a GEMV with one
         // atomicMax per workgroup and a copy of the key)
         GemvArgs g = gemv_args(h);
         g.xf = x; g.gamma = h->g_final; g.w = h->lm_w; g.ws = h->lm_s; g.y = logits; g.n = V; g.k = D;
